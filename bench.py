@@ -222,7 +222,11 @@ def main(argv=None) -> int:
         kernel, avg_ms, alg_bytes = "k_yee_e3", e_ms, bytes_e
     else:
         kernel, avg_ms, alg_bytes = "k_yee_h3", h_ms, bytes_h
-    if "pml_split=1" in eng.describe():
+    one_pass = " step3=1" in eng.describe()
+    if one_pass:  # H and E in one launch, timed as the E pass: 12 values and one id a cell
+        kernel, avg_ms = "k_step3", e_ms
+        alg_bytes = cells * (12 * sbytes + id_bytes) + pml_bytes(sim, "h", cbytes) + pml_bytes(sim, "e", cbytes)
+    elif "pml_split=1" in eng.describe():
         kernel += "+k_pml_z"  # the pass: Yee kernel, then its z-face CPML launch
     achieved = alg_bytes / (avg_ms * 1e-3) / 1e9
     traffic = None
@@ -395,6 +399,10 @@ def bench_batch(args) -> int:
         kernel, avg_ms, alg_bytes = "k_yee_e3_batch", e_ms, bytes_e
     else:
         kernel, avg_ms, alg_bytes = "k_yee_h3_batch", h_ms, bytes_h
+    if " step3=1" in desc:  # H and E in one launch, timed as the E pass
+        kernel, avg_ms = "k_step3", e_ms
+        alg_bytes = sum(int(np.prod(s.info()[0])) * (12 * sbytes + 1) + pml_bytes(s, "h", cbytes) +
+                        pml_bytes(s, "e", cbytes) for s in sims)
     achieved = alg_bytes / (avg_ms * 1e-3) / 1e9
 
     accuracy = batch_far_field(args, prec, w16) if args.full_steps > 0 else None
@@ -710,6 +718,9 @@ def bench_fp32_vs_fp64(args) -> int:
         e_ms = tm["yee_e_ms"] / tm["yee_e_launches"]
         kname = ("k_yee_e2" if two_d else
                  ("k_yee_e3+k_pml_z+k_ade_e3" if "pml_split=1" in desc else "k_yee_e3+k_ade_e3"))
+        if " step3=1" in desc:  # H and E in one launch, timed (with the ADE kernel) as the E pass
+            kname = "k_step3+k_ade_e3"
+            e_bytes = ncell * (12 * sb + 1) + pml_bytes(sim, "h", cb) + pml_bytes(sim, "e", cb)
         out["roofline"] = {"bound": "hbm", "kernel": kname,
                            "achieved": round(e_bytes / (e_ms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBPS,
                            "unit": "GB/s",
@@ -720,7 +731,7 @@ def bench_fp32_vs_fp64(args) -> int:
                            "avg_launch_ms": round(e_ms, 5), "h_ms": round(tm["yee_h_ms"] / tm["yee_h_launches"], 5),
                            "post_h_ms": round(tm["tfsf_ms"] / 10, 5), "post_e_ms": round(tm["nf2ff_ms"] / 10, 5),
                            "note": ("E pass events (the Yee kernel with its CPML, plus the ADE kernel "
-                                    "in 3-D; on 2-D FP64/FP32 grids the TF/SF corrections run inside "
+                                    "in 3-D, where one launch does H and E; on 2-D FP64/FP32 grids the TF/SF corrections run inside "
                                     "k_yee_h2/k_yee_e2); algorithmic bytes count the fields, ids and "
                                     "psi, not the ADE J arrays. post_h_ms / post_e_ms: what follows "
                                     "each pass (TF/SF launches where not fused, sources, NF2FF, movies)") }

@@ -1,6 +1,8 @@
 """In-tree build of the package's native code (python -m xfdtd_cuda_amd.build).
 
-libxfdtd_hip.so  hipcc --offload-arch=gfx950: the time-stepping engine.
+libxfdtd_hip.so  hipcc --offload-arch=gfx950: the time-stepping engine, and
+                 its one-pass step once per storage type, compiled at the
+                 same time.
 libxfdtd_host.so g++: scene set-up, SimulationHD drop-in, C ABI for Python.
 tests/cpp/simulation_hd_driver  g++: the C++ drop-in driver test.
 
@@ -13,6 +15,8 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -20,7 +24,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 CXX = os.environ.get("CXX", "g++")
 
 HIP_FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off",
+    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wall",
 ]
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-fopenmp", "-Wall", "-Wextra",
@@ -39,10 +43,21 @@ def _run(cmd, cwd):
         raise RuntimeError(f"build step failed ({r.returncode}): {' '.join(cmd)}")
 
 
+# storage types of the one-pass step (csrc/xf_step3.hip, a translation unit each)
+STEP3_STORES = ("double", "float", "__half", "__hip_bfloat16", "Bf16c")
+
+
 def build_hip():
-    src = os.path.join(HERE, "csrc", "xf_engine.hip")
     out = os.path.join(HERE, "libxfdtd_hip.so")
-    _run([HIPCC, *HIP_FLAGS, "-o", out + ".tmp", src], HERE)
+    csrc = os.path.join(HERE, "csrc")
+    with tempfile.TemporaryDirectory(prefix="_build", dir=HERE) as tmp:
+        units = [("xf_engine.hip", "engine.o", [])]
+        units += [("xf_step3.hip", f"step3_{s}.o", [f"-DXF_STEP3_STORE={s}"]) for s in STEP3_STORES]
+        with ThreadPoolExecutor(min(len(units), os.cpu_count() or 1)) as pool:
+            list(pool.map(lambda u: _run([HIPCC, *HIP_FLAGS, *u[2], "-c", "-o", os.path.join(tmp, u[1]),
+                                          os.path.join(csrc, u[0])], HERE), units))
+        _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out + ".tmp",
+              *(os.path.join(tmp, u[1]) for u in units)], HERE)
     os.replace(out + ".tmp", out)
 
 

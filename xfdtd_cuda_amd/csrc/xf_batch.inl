@@ -40,6 +40,8 @@ struct Batch {
   int64_t* tf_start[2]{};
   int n_tf[2]{0, 0};
   int64_t tf_total[2]{0, 0};
+  // NF2FF, point-source and learned-layer items of fields in either set of the
+  // one-pass step (two arrays, one after the other)
   void* nf_items{};
   int64_t* nf_start{};
   int n_nf{0};
@@ -59,8 +61,21 @@ struct Batch {
   int64_t lb_blocks{0}, lb_mblocks{0};
   bool lb_any_record{false};
   int* t_dev{};
-  hipGraph_t graph{};
-  hipGraphExec_t graph_exec{};
+  // the one-pass step of every grid in one launch (each grid's blocks in turn)
+  bool step3_auto{true};  // the tiling was left to the engine
+  void* step3_desc{};     // [2][grids] Step3Pass
+  int* step3_start{};
+  int step3_blocks{0};
+  size_t step3_lds{0};
+  bool step3_pml{false};
+  bool step3_fits{false};
+  bool use_step3() const { return step3_auto && step3_fits; }
+  int set() const { return inst.empty() ? 0 : inst[0]->eng.step3_set; }
+  void swap_sets() {
+    for (auto& h : inst) h->eng.step3_swap();
+  }
+  hipGraph_t graph[2]{};
+  hipGraphExec_t graph_exec[2]{};
   bool graph_ready{false};
   xf_timing timing{};
   std::string desc;
@@ -68,10 +83,12 @@ struct Batch {
   ~Batch() { release(); }
 
   void drop_graph() {
-    if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
-    if (graph) (void)hipGraphDestroy(graph);
-    graph_exec = nullptr;
-    graph = nullptr;
+    for (int q = 0; q < 2; ++q) {
+      if (graph_exec[q]) (void)hipGraphExecDestroy(graph_exec[q]);
+      if (graph[q]) (void)hipGraphDestroy(graph[q]);
+      graph_exec[q] = nullptr;
+      graph[q] = nullptr;
+    }
     graph_ready = false;
   }
 
@@ -83,6 +100,9 @@ struct Batch {
     tile_start = nullptr;
     tf_items[0] = tf_items[1] = nf_items = pt_items = lb_items = nullptr;
     tf_start[0] = tf_start[1] = nf_start = lb_bstart = lb_mstart = lb_estart = nullptr;
+    step3_desc = nullptr;
+    step3_start = nullptr;
+    step3_fits = false;
     pz_items[0] = pz_items[1] = nullptr;
     pz_start[0] = pz_start[1] = nullptr;
     t_dev = nullptr;
@@ -303,9 +323,55 @@ int Batch::configure_t() {
     XF_TRY(put(&q, st.data(), st.size() * sizeof(int64_t)));
     tf_start[pass] = static_cast<int64_t*>(q);
   }
+  // the one-pass step: descriptors of both directions, the blocks of all
+  // grids in turn
+  step3_fits = true;
+  for (int g = 0; g < n; ++g) step3_fits = step3_fits && eng(g).step3_ready;
+  if (step3_fits) {
+    std::vector<Step3Pass<S>> desc(2 * static_cast<size_t>(n));
+    std::vector<int> start(n + 1, 0);
+    int64_t blocks = 0;
+    step3_lds = 0;
+    step3_pml = false;
+    for (int g = 0; g < n; ++g) {
+      Engine& E = eng(g);
+      step3_lds = std::max(step3_lds, E.step3_lds());
+      step3_pml = step3_pml || !E.pml.empty();
+    }
+    std::vector<const Engine*> grids;
+    for (int g = 0; g < n; ++g) grids.push_back(&eng(g));
+    const int chunk = step3_pick_chunk<S>(grids, step3_pml, step3_lds);
+    for (int g = 0; g < n; ++g) eng(g).step3_chunk = chunk;
+    for (int s = 0; s < 2; ++s) {
+      for (int g = 0; g < n; ++g) desc[static_cast<size_t>(eng(g).step3_set) * n + g] = eng(g).template step3_pass<S>();
+      swap_sets();
+    }
+    for (int g = 0; g < n; ++g) {
+      start[g] = static_cast<int>(blocks);
+      blocks += static_cast<int64_t>(desc[g].nkb) * desc[g].njb * desc[g].nch;
+      if (blocks > INT_MAX / 2) return fail(XF_ERR_UNSUPPORTED, "batch too large for 32-bit block ids");
+    }
+    start[n] = step3_blocks = static_cast<int>(blocks);
+    XF_TRY(put(&step3_desc, desc.data(), desc.size() * sizeof(Step3Pass<S>)));
+    void* q = step3_start;
+    XF_TRY(put(&q, start.data(), start.size() * sizeof(int)));
+    step3_start = static_cast<int*>(q);
+  }
+  // Items of the current set, then of the other (where there is one): set
+  // s's are at [s] of the two halves.
+  auto both = [&](auto&& build) {
+    const int sets = step3_fits ? 2 : 1;
+    for (int s = 0; s < sets; ++s) {
+      build(set());
+      if (sets == 2) swap_sets();
+    }
+  };
   {
-    std::vector<NfItem<S>> items;
-    std::vector<int64_t> st(1, 0);
+    std::vector<NfItem<S>> halves[2], &items = halves[0];
+    std::vector<int64_t> st;
+    both([&](int s) {
+    std::vector<NfItem<S>>& items = halves[s];
+    st.assign(1, 0);
     for (int g = 0; g < n; ++g) {
       Engine& E = eng(g);
       for (auto& N : E.nf) {
@@ -319,7 +385,9 @@ int Batch::configure_t() {
         st.push_back(st.back() + whole_blocks(N.pass.total));
       }
     }
-    n_nf = static_cast<int>(items.size());
+    });
+    halves[0].insert(halves[0].end(), halves[1].begin(), halves[1].end());
+    n_nf = static_cast<int>(st.size()) - 1;
     nf_total = st.back();
     XF_TRY(put(&nf_items, items.data(), items.size() * sizeof(NfItem<S>)));
     void* q = nf_start;
@@ -328,7 +396,9 @@ int Batch::configure_t() {
   }
   // point sources and learned layers
   {
-    std::vector<PointItem<S>> items;
+    std::vector<PointItem<S>> halves[2], &items = halves[0];
+    both([&](int s) {
+    n_pt = 0;
     for (int g = 0; g < n; ++g) {
       Engine& E = eng(g);
       if (E.pts.n == 0) continue;
@@ -336,15 +406,21 @@ int Batch::configure_t() {
       it.f = make_fields<S>(E);
       it.sc = make_scales<C>(E);
       it.P = E.pts;
-      items.push_back(it);
+      halves[s].push_back(it);
+      ++n_pt;
     }
-    n_pt = static_cast<int>(items.size());
+    });
+    halves[0].insert(halves[0].end(), halves[1].begin(), halves[1].end());
     XF_TRY(put(&pt_items, items.data(), items.size() * sizeof(PointItem<S>)));
   }
   {
-    std::vector<LbItem<S>> items;
-    std::vector<int64_t> st(1, 0), sm(1, 0), se(1, 0);
+    std::vector<LbItem<S>> halves[2], &items = halves[0];
+    std::vector<int64_t> st, sm, se;
     lb_any_record = false;
+    both([&](int s) {
+    st.assign(1, 0);
+    sm.assign(1, 0);
+    se.assign(1, 0);
     for (int g = 0; g < n; ++g) {
       Engine& E = eng(g);
       if (!E.has_lb || E.lbd.total == 0) continue;
@@ -353,15 +429,17 @@ int Batch::configure_t() {
       it.sc = make_scales<C>(E);
       it.d = make_dims(E);
       it.L = E.lbd;
-      items.push_back(it);
+      halves[s].push_back(it);
       st.push_back(st.back() + (E.lbd.total + 255) / 256);
       const bool apply = E.lbd.mode == XF_LB_APPLY;
       sm.push_back(sm.back() + (apply ? (E.lbd.total + kLbMfmaCols - 1) / kLbMfmaCols : 0));
       se.push_back(se.back() + (apply ? E.lbd.n_edge : 0));
       lb_any_record = lb_any_record || !apply;
     }
+    });
+    halves[0].insert(halves[0].end(), halves[1].begin(), halves[1].end());
     lb_edges = se.back();
-    n_lb = static_cast<int>(items.size());
+    n_lb = static_cast<int>(st.size()) - 1;
     lb_blocks = st.back();
     lb_mblocks = sm.back();
     if (lb_blocks > INT_MAX) return fail(XF_ERR_UNSUPPORTED, "learned layers too large for one launch");
@@ -413,7 +491,8 @@ int Batch::configure() {
          " pml_ztail=" + std::to_string(tune.pml_split == 2 ? 1 : 0) +
          " k32=" + std::to_string(tune.k32) + " xcd=" + std::to_string(tune.xcd_remap) +
          " tfsf=" + std::to_string(n_tf[0]) +
-         " nf2ff=" + std::to_string(n_nf) + " cpsi_tab=" + std::to_string(cpsi_tab);
+         " nf2ff=" + std::to_string(n_nf) + " cpsi_tab=" + std::to_string(cpsi_tab) +
+         " step3=" + std::to_string(use_step3() ? 1 : 0) + (use_step3() ? " step3_blocks=" + std::to_string(step3_blocks) : std::string());
   return XF_OK;
 }
 
@@ -441,6 +520,14 @@ int Batch::launch_step(int t, bool use_tdev, bool ev_on, hipEvent_t* ev) {
     if (id_bytes == 1) XF_BYLV(KER, uint8_t, PASS); else XF_BYLV(KER, uint16_t, PASS);         \
   } while (0)
   if (ev_on) XF_HIP(hipEventRecord(ev[0], stream));
+  if (use_step3()) {
+    if (ev_on) XF_HIP(hipEventRecord(ev[1], stream));
+    if (ev_on) XF_HIP(hipEventRecord(ev[2], stream));
+    XF_HIP(step3_launch<S>(static_cast<const Step3Pass<S>*>(step3_desc) + static_cast<size_t>(set()) * n, step3_start, n,
+                           step3_blocks, step3_pml, step3_lds, t, tp, stream));
+    swap_sets();
+    if (ev_on) XF_HIP(hipEventRecord(ev[3], stream));
+  } else {
   XF_BYALL(k_yee_h3_batch, pass_h);
   if (pz_total[0] > 0)
     hipLaunchKernelGGL((k_pml_z_batch<S, false>), dim3((unsigned)((pz_total[0] + 255) / 256)), dim3(256), 0,
@@ -458,15 +545,18 @@ int Batch::launch_step(int t, bool use_tdev, bool ev_on, hipEvent_t* ev) {
   if (tf_total[1] > 0)
     hipLaunchKernelGGL((k_tfsf_batch<S>), dim3((unsigned)((tf_total[1] + 255) / 256)), dim3(256), 0, stream,
                        static_cast<const TfsfItem<S>*>(tf_items[1]), tf_start[1], n_tf[1], t, tp);
+  }
+  // the items of the set the fields are in now
+  const size_t half = step3_fits ? static_cast<size_t>(set()) : 0;
   // per grid: point sources, then the learned layer's phases, then movies,
   // as Engine::launch_additions orders them; the grids share no memory
   if (n_pt > 0)
     hipLaunchKernelGGL((k_point_sources_batch<S>), dim3((unsigned)((n_pt + 63) / 64)), dim3(64), 0, stream,
-                       static_cast<const PointItem<S>*>(pt_items), n_pt, t, tp);
+                       static_cast<const PointItem<S>*>(pt_items) + half * n_pt, n_pt, t, tp);
   if (n_lb > 0) {
     // phase 0 (RECORD layers on the VALU, APPLY layers on the matrix
     // cores), the edge nodes of APPLY layers, the history roll
-    const LbItem<S>* li = static_cast<const LbItem<S>*>(lb_items);
+    const LbItem<S>* li = static_cast<const LbItem<S>*>(lb_items) + half * n_lb;
     // recording layers: phase 0 (record) and 2 (roll) over all columns;
     // apply layers: the network with the roll of its columns, then the edge
     // columns' Mur update and roll
@@ -487,7 +577,7 @@ int Batch::launch_step(int t, bool use_tdev, bool ev_on, hipEvent_t* ev) {
   for (auto& h : inst) XF_TRY(h->eng.launch_movies<S>(t, tp, stream));
   if (nf_total > 0)
     hipLaunchKernelGGL((k_nf2ff_batch<S>), dim3((unsigned)((nf_total + 255) / 256)), dim3(256), 0, stream,
-                       static_cast<const NfItem<S>*>(nf_items), nf_start, n_nf, t, tp);
+                       static_cast<const NfItem<S>*>(nf_items) + half * n_nf, nf_start, n_nf, t, tp);
   for (auto& h : inst) XF_TRY(h->eng.launch_td<S>(t, tp, stream));
   if (ev_on) XF_HIP(hipEventRecord(ev[4], stream));
   if (use_tdev) hipLaunchKernelGGL(k_next_step, dim3(1), dim3(1), 0, stream, t_dev);
@@ -544,10 +634,22 @@ int Batch::run(int64_t n) {
     for (auto& h : inst) hipLaunchKernelGGL(k_watch_clear, dim3(1), dim3(64), 0, stream, h->eng.wd_dev);
   if (graph_on) {
     if (!graph_ready) {
-      XF_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-      const int st = step(0, true, false, nullptr);
-      XF_TRY(end_capture(stream, st, &graph));
-      XF_HIP(hipGraphInstantiate(&graph_exec, graph, nullptr, nullptr, 0));
+      // as Engine::run: a graph per set of the one-pass step
+      drop_graph();
+      const int set0 = set(), n_graph = use_step3() ? 2 : 1;
+      auto failed = [&](int st) {
+        if (set() != set0) swap_sets();
+        return st;
+      };
+      for (int q = 0; q < n_graph; ++q) {
+        const int slot = use_step3() ? set() : 0;
+        XF_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+        const int st = end_capture(stream, step(0, true, false, nullptr), &graph[slot]);
+        if (st != XF_OK) return failed(st);
+        const hipError_t made = hipGraphInstantiate(&graph_exec[slot], graph[slot], nullptr, nullptr, 0);
+        if (made != hipSuccess)
+          return failed(fail(XF_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(made)));
+      }
       graph_ready = true;
     }
     const int t0 = static_cast<int>(cur_step);
@@ -555,7 +657,8 @@ int Batch::run(int64_t n) {
     XF_HIP(hipStreamSynchronize(stream));
     XF_HIP(hipEventRecord(run0, stream));
     for (int64_t s = 0; s < n; ++s) {
-      XF_HIP(hipGraphLaunch(graph_exec, stream));
+      XF_HIP(hipGraphLaunch(graph_exec[use_step3() ? set() : 0], stream));
+      if (use_step3()) swap_sets();
       if (wd && ((cur_step + s + 1) % wd == 0 || s + 1 == n)) XF_TRY(watch(s + 1));
     }
   } else {
@@ -602,7 +705,7 @@ int Batch::run(int64_t n) {
   }
   // algorithmic bytes per cell-step, cell-weighted over the grids
   double bytes = 0;
-  for (auto& h : inst) bytes += h->eng.bytes_per_cell_step() * static_cast<double>(h->eng.nx * h->eng.ny * h->eng.nz);
+  for (auto& h : inst) bytes += h->eng.bytes_per_cell_step(use_step3()) * static_cast<double>(h->eng.nx * h->eng.ny * h->eng.nz);
   timing.bytes_per_cell_step = bytes / static_cast<double>(cells);
   cur_step += n;
   sync_steps();
@@ -658,7 +761,27 @@ int Batch::autotune(int trial_steps, xf_tuning* best) {
     h->eng.pml_split = keep_split;
     h->eng.pml_ztail = keep_tail;
   }
+  // the one-pass step, then the two-pass tilings
+  const bool keep_auto = step3_auto;
+  bool win_step3 = false;
+  step3_auto = true;
+  if (step3_fits) {
+    tune = xf_tuning{1, 4, 0, 1, 0, 1, 0, 0.0};
+    status = configure();
+    if (status == XF_OK) status = run(1);
+    if (status == XF_OK) status = run(trial_steps);
+    if (status == XF_OK) {
+      win = tune;
+      win.step_ms = timing.run_ms / trial_steps;
+      win_step3 = true;
+      cur_step = step0;
+      sync_steps();
+      status = restore();
+    }
+  }
+  step3_auto = false;
   for (int ty : {1, 2, 4}) {
+    if (status != XF_OK) break;
     // 6 planes: 30.29 against 30.08-30.11 Gcells/s for 4 on the FP32 64-grid
     // batch at the tuner's other choices (5: 30.36, 3: 29.66)
     for (int planes : {2, 4, 6, 8, 16}) {
@@ -681,6 +804,7 @@ int Batch::autotune(int trial_steps, xf_tuning* best) {
           if (ms < win.step_ms) {
             win = tune;
             win.step_ms = ms;
+            win_step3 = false;
           }
           cur_step = step0;
           sync_steps();
@@ -697,6 +821,7 @@ int Batch::autotune(int trial_steps, xf_tuning* best) {
   timing = keep;
   cur_step = step0;
   sync_steps();
+  step3_auto = status == XF_OK ? win_step3 : keep_auto;
   if (status != XF_OK) {
     (void)restore();
     return status;
@@ -732,7 +857,21 @@ int Engine::autotune(int trial_steps, xf_tuning* best) {
   const bool can_tail = ztail();
   pml_split = keep_split;
   pml_ztail = keep_tail;
+  // the one-pass step, then the two-pass tilings
+  bool win_step3 = false;
+  if (step3_ready) {
+    set_tiling(0, 0, 0);
+    status = run(1);
+    if (status == XF_OK) status = run(trial_steps);
+    if (status == XF_OK) {
+      win = xf_tuning{1, step3_chunk, 0, 1, 0, 0, 0, timing.run_ms / trial_steps};
+      win_step3 = true;
+      cur_step = step0;
+      status = restore();
+    }
+  }
   for (int ty : tys) {
+    if (status != XF_OK) break;
     for (int planes : pls) {
       for (int nt_on : {1, 0}) {
         for (int cand = 0; cand < 6; ++cand) {
@@ -746,7 +885,10 @@ int Engine::autotune(int trial_steps, xf_tuning* best) {
           if (status == XF_OK) status = run(trial_steps);
           if (status != XF_OK) break;
           const double ms = timing.run_ms / trial_steps;
-          if (ms < win.step_ms) win = xf_tuning{ty, planes, 0, nt_on, 0, split, k32, ms};
+          if (ms < win.step_ms) {
+            win = xf_tuning{ty, planes, 0, nt_on, 0, split, k32, ms};
+            win_step3 = false;
+          }
           cur_step = step0;
           status = restore();
           if (status != XF_OK) break;
@@ -764,10 +906,14 @@ int Engine::autotune(int trial_steps, xf_tuning* best) {
     (void)restore();
     return status;
   }
+  if (best) *best = win;
+  if (win_step3) {
+    set_tiling(0, 0, 0);
+    return XF_OK;
+  }
   set_tiling(win.tile_y, static_cast<int>((nx + 1 + win.planes - 1) / win.planes),
              XF_TILE_SET | (win.nontemporal ? XF_TILE_NT : 0) | (win.pml_split == 1 ? XF_TILE_PML_SPLIT : 0) |
                  (win.pml_split == 2 ? XF_TILE_PML_ZTAIL : 0) | (win.k32 ? XF_TILE_K32 : 0));
-  if (best) *best = win;
   return XF_OK;
 }
 
@@ -839,16 +985,20 @@ int xf_batch_set_tuning(xf_batch* b, const xf_tuning* t) {
     xf::g_err.clear();
     if (!b || !t) return xf::fail(XF_ERR_INVALID, "null argument");
     const xf_tuning keep = b->b.tune;
+    const bool keep_auto = b->b.step3_auto;
     b->b.tune = *t;
     b->b.tune.step_ms = 0;
+    b->b.step3_auto = false;
     if (t->tile_y < 1 || t->tile_y > 4 || t->planes < 1 || t->blocks < 0 || t->pml_split < 0 || t->pml_split > 2) {
       b->b.tune = keep;
+      b->b.step3_auto = keep_auto;
       return xf::fail(XF_ERR_INVALID, "bad tuning (tile_y 1..4, planes >= 1, blocks >= 0, pml_split 0..2)");
     }
     if (!b->b.uploaded) return XF_OK;
     const int st = b->b.configure();
     if (st != XF_OK) {
       b->b.tune = keep;
+      b->b.step3_auto = keep_auto;
       (void)b->b.configure();
     }
     return st;

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <numeric>
 #include <array>
 #include <cmath>
 #include <cstring>
@@ -165,6 +166,56 @@ struct Engine {
   std::vector<void*> backup;
   // fields
   void* fld[6]{};
+  // The one-pass 3-D step (k_step3) reads fld and the H pass's psi and
+  // writes a second set, fld2 and PmlDev::psi2; the sets are swapped after
+  // each launch, so fld and psi always name the current ones.  step3_set
+  // counts the swaps modulo two: the descriptor a launch takes.
+  void* fld2[6]{};
+  bool step3_ready{false};  // the scene has the one-pass form (tables and second set on the device)
+  bool step3_auto{true};    // the tiling was left to the engine
+  int step3_set{0};
+  void* step3_ids{};        // one byte per node: row of step3_tab
+  void* step3_tab{};        // 18 coefficients per pair of E and H rows
+  int step3_rows{0};
+  uint64_t step3_dmask{0};
+  void* step3_desc{};       // two Step3Pass, one per direction
+  int* step3_start{};
+  int step3_blocks{0}, step3_chunk{1};
+  // One pass wherever the scene has the form (step3_tables, step3_incident,
+  // step3_faces): on the grids measured it is the faster one or even, us a
+  // step against two passes: 536^3 FP64 3765 / 4730, 148^3 FP64 167 / 204,
+  // 50^3 FP64 the least, 253^3 FP32 420 / 419, FP16 storage 423 / 483.
+  bool use_step3() const { return step3_ready && step3_auto; }
+  void step3_swap() {
+    std::swap_ranges(fld, fld + 6, fld2);
+    for (PmlDev& D : pml) {
+      std::swap(D.psi[2], D.psi2[0]);
+      std::swap(D.psi[3], D.psi2[1]);
+    }
+    step3_set ^= 1;
+  }
+  // where a state buffer's contents are now (the two sets are one state)
+  void* live(void* p) {
+    for (int c = 0; c < 6; ++c)
+      if (p && (p == fld[c] || p == fld2[c])) return fld[c];
+    for (PmlDev& D : pml)
+      for (int q = 0; q < 2; ++q)
+        if (p == D.psi[2 + q] || p == D.psi2[q]) return D.psi[2 + q];
+    return p;
+  }
+  int step3_tables(const std::vector<uint32_t>& ide, const std::vector<uint32_t>& idh);
+  bool step3_incident() const;
+  bool step3_faces() const;
+  int step3_alloc();
+  template <typename S>
+  Step3Pass<S> step3_pass() const;
+  template <typename S>
+  int step3_describe();
+  size_t step3_lds() const { return static_cast<size_t>(step3_rows) * 18 * (plan.precision == XF_FP64 ? 8 : 4); }
+  template <typename S>
+  int launch_step3(int t, const int* tp);
+  template <typename S>
+  int launch_ade(hipStream_t st);
   // coefficient ids and tables (compute type)
   void* eid{};
   void* hid{};
@@ -191,6 +242,7 @@ struct Engine {
     void *ca_e, *cb_e, *ca_h, *cb_h;
     void* cpsi[4];
     void* psi[4];
+    void* psi2[2];  // the H pass's psi (2, 3), other set
   };
   std::vector<PmlDev> pml;
   // TFSF
@@ -235,9 +287,18 @@ struct Engine {
   unsigned* wd_dev{};
   template <typename S>
   int launch_watch(int64_t step, hipStream_t st);
-  hipGraph_t graph{};
-  hipGraphExec_t graph_exec{};
+  hipGraph_t graph[2]{};  // one step from each set of the one-pass step; else only the first
+  hipGraphExec_t graph_exec[2]{};
   bool graph_ready{false};
+  void drop_graph() {
+    for (int q = 0; q < 2; ++q) {
+      if (graph_exec[q]) (void)hipGraphExecDestroy(graph_exec[q]);
+      if (graph[q]) (void)hipGraphDestroy(graph[q]);
+      graph_exec[q] = nullptr;
+      graph[q] = nullptr;
+    }
+    graph_ready = false;
+  }
   // timing
   xf_timing timing{};
   int tile_y{4};
@@ -281,15 +342,16 @@ struct Engine {
   ~Engine() { release(); }
 
   void release() {
-    if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
-    if (graph) (void)hipGraphDestroy(graph);
-    graph_exec = nullptr;
-    graph = nullptr;
-    graph_ready = false;
+    drop_graph();
     for (void* p : allocs) (void)hipFree(p);
     allocs.clear();
     state.clear();
     backup.clear();
+    std::fill(fld2, fld2 + 6, nullptr);
+    step3_ready = false;
+    step3_set = 0;
+    step3_ids = step3_tab = step3_desc = nullptr;
+    step3_start = nullptr;
     if (stream) (void)hipStreamDestroy(stream);
     stream = nullptr;
     if (stream2) (void)hipStreamDestroy(stream2);
@@ -399,7 +461,7 @@ struct Engine {
   template <typename S>
   int launch_td(int t, const int* tp, hipStream_t st);
 
-  double bytes_per_cell_step() const;
+  double bytes_per_cell_step(bool one_pass) const;
 };
 
 // ------------------------------------------------------------ validation
@@ -933,9 +995,11 @@ int Engine::check_ade_pml() const {
   return XF_OK;
 }
 
-double Engine::bytes_per_cell_step() const {
+double Engine::bytes_per_cell_step(bool one_pass) const {
   // H pass: read H3 + E3, write H3; E pass: read E3 + H3, write E3, plus one
-  // coefficient index per pass.
+  // coefficient index per pass.  The one-pass step reads and writes the six
+  // components once, with one index.
+  if (one_pass) return 12.0 * static_cast<double>(esize) + 1.0;
   const double fields = 2.0 * 9.0 * static_cast<double>(esize);
   return fields + 2.0 * id_bytes;
 }
@@ -1235,7 +1299,127 @@ int Engine::build_ids() {
           if (disp[(i * ny + j) * nz + k]) ade_cells.push_back((i * (ny + 1) + j) * (nz + 1) + k);
   }
   match_cpsi(ide, idh);
-  return XF_OK;
+  return step3_tables(ide, idh);
+}
+
+// The one-pass step's ids: the pairs of E and H rows that occur, (0, 0)
+// first (a node that is no cell has row 0 in both tables).  Its blocks hold
+// the whole table in LDS, so a scene with more than kStep3MaxRows pairs, or
+// dense coefficients, keeps the two-pass kernels.
+int Engine::step3_tables(const std::vector<uint32_t>& ide, const std::vector<uint32_t>& idh) {
+  step3_rows = 0;
+  if (dense || dim != 3 || sy >= (int64_t(1) << 24) || ntab_e > kStep3MaxRows || ntab_h > kStep3MaxRows) return XF_OK;
+  const size_t most = has_ade ? kStep3AdeRows : kStep3MaxRows;
+  std::vector<int> at(static_cast<size_t>(ntab_e) * ntab_h, -1);
+  std::vector<std::pair<int, int>> pairs{{0, 0}};
+  at[0] = 0;
+  const int64_t cells = nx * ny * nz;
+  int64_t run_end = 0;
+  uint32_t le = 0, lh = 0;
+  std::vector<uint8_t> id(static_cast<size_t>(cells));
+  for (int64_t c = 0; c < cells; ++c) {
+    if (c == 0 || ide[c] != le || idh[c] != lh) {
+      le = ide[c];
+      lh = idh[c];
+      int& p = at[static_cast<size_t>(le) * ntab_h + lh];
+      if (p < 0) {
+        if (pairs.size() >= most) return XF_OK;
+        p = static_cast<int>(pairs.size());
+        pairs.emplace_back(static_cast<int>(le), static_cast<int>(lh));
+      }
+      run_end = p;
+    }
+    id[c] = static_cast<uint8_t>(run_end);
+  }
+  std::vector<double> tab;
+  step3_dmask = 0;
+  for (size_t q = 0; q < pairs.size(); ++q) {
+    for (int n = 0; n < 9; ++n) tab.push_back(etab_h[static_cast<size_t>(pairs[q].first) * 9 + n]);
+    for (int n = 0; n < 9; ++n) tab.push_back(htab_h[static_cast<size_t>(pairs[q].second) * 9 + n]);
+    if (has_ade && eflag_h[pairs[q].first]) step3_dmask |= uint64_t(1) << q;
+  }
+  XF_TRY(upload_c(&step3_tab, tab.data(), static_cast<int64_t>(tab.size())));
+  step3_rows = static_cast<int>(pairs.size());
+  std::vector<uint8_t> v(total, 0);
+  for (int64_t i = 0; i < nx; ++i)
+    for (int64_t j = 0; j < ny; ++j)
+      std::copy_n(id.data() + (i * ny + j) * nz, nz, v.data() + i * sx + j * sy);
+  return upload_vec(&step3_ids, v);
+}
+
+// Whether a block's share of the incident tables is bounded as k_step3 holds
+// it: projections that change by at most 1.5 a node, the same way along each
+// axis (a plane wave's change by less than 1.2), and half-grid ones beside them.
+bool Engine::step3_incident() const {
+  if (!sc->tfsf) return true;
+  const xf_tfsf& T = *sc->tfsf;
+  const xf_array* pi[3] = {&T.proj_x_int, &T.proj_y_int, &T.proj_z_int};
+  const xf_array* ph[3] = {&T.proj_x_half, &T.proj_y_half, &T.proj_z_half};
+  for (int d = 0; d < 3; ++d) {
+    if (pi[d]->shape[0] != ph[d]->shape[0] || pi[d]->shape[0] < 1) return false;
+    for (const xf_array* a : {pi[d], ph[d]}) {
+      const double dir = a->data[a->shape[0] - 1] - a->data[0];
+      for (int64_t q = 0; q + 1 < a->shape[0]; ++q) {
+        const double s = a->data[q + 1] - a->data[q];
+        if (!(std::fabs(s) <= 1.5) || s * dir < 0) return false;
+      }
+    }
+    for (int64_t q = 0; q < pi[d]->shape[0]; ++q)
+      if (!(std::fabs(pi[d]->data[q] - ph[d]->data[q]) <= 1.0)) return false;
+  }
+  return true;
+}
+
+// The second set of fields and H-pass psi, a copy of the first, where it
+// takes at most a quarter of the device memory that is free (the rest is left
+// to other engines and to the caller); without it the two-pass kernels run.
+int Engine::step3_alloc() {
+  if (step3_rows == 0 || !step3_incident() || !step3_faces()) return XF_OK;
+  const size_t kept = allocs.size();
+  bool fits = true;
+  auto second = [&](void** p, size_t bytes) {
+    *p = nullptr;
+    if (!fits) return;
+    if (hipMalloc(p, bytes ? bytes : 16) != hipSuccess) {
+      (void)hipGetLastError();
+      *p = nullptr;
+      fits = false;
+      return;
+    }
+    allocs.push_back(*p);
+  };
+  auto psi_bytes = [&](size_t q, int c) {
+    const xf_pml& P = sc->pml[pml_order[q]];
+    return static_cast<size_t>(numel(c == 0 ? P.ha_psi_eb : P.hb_psi_ea)) * (plan.precision == XF_FP64 ? 8 : 4);
+  };
+  size_t want = 6 * static_cast<size_t>(total) * esize, free_bytes = 0, all_bytes = 0;
+  for (size_t q = 0; q < pml.size(); ++q) want += psi_bytes(q, 0) + psi_bytes(q, 1);
+  XF_HIP(hipMemGetInfo(&free_bytes, &all_bytes));
+  if (want > free_bytes / 4) return XF_OK;
+  for (int c = 0; c < 6; ++c) second(&fld2[c], static_cast<size_t>(total) * esize);
+  for (size_t q = 0; q < pml.size(); ++q)
+    for (int c = 0; c < 2; ++c) second(&pml[q].psi2[c], psi_bytes(q, c));
+  if (!fits) {
+    for (size_t q = kept; q < allocs.size(); ++q) (void)hipFree(allocs[q]);
+    allocs.resize(kept);
+    std::fill(fld2, fld2 + 6, nullptr);
+    for (PmlDev& D : pml) D.psi2[0] = D.psi2[1] = nullptr;
+    return XF_OK;
+  }
+  for (int c = 0; c < 6; ++c)
+    XF_HIP(hipMemcpyAsync(fld2[c], fld[c], static_cast<size_t>(total) * esize, hipMemcpyDeviceToDevice, stream));
+  for (size_t q = 0; q < pml.size(); ++q)
+    for (int c = 0; c < 2; ++c)
+      XF_HIP(hipMemcpyAsync(pml[q].psi2[c], pml[q].psi[2 + c], psi_bytes(q, c), hipMemcpyDeviceToDevice, stream));
+  XF_HIP(hipStreamSynchronize(stream));
+  step3_ready = true;
+  switch (plan.precision) {
+    case XF_FP64: return step3_describe<double>();
+    case XF_FP32: return step3_describe<float>();
+    case XF_BF16_COMP: return step3_describe<Bf16c>();
+    case XF_FP16_STORE: return step3_describe<__half>();
+    default: return step3_describe<__hip_bfloat16>();
+  }
 }
 
 // The c_psi value of a corrected node is the curl coefficient, along the
@@ -1816,6 +2000,7 @@ int Engine::upload() {
   t_dev = static_cast<int*>(tp);
   XF_TRY(alloc(&tp, 64));
   wd_dev = static_cast<unsigned*>(tp);
+  XF_TRY(step3_alloc());
   set_tiling(plan.tile_y, plan.chunks_x, plan.tiling_flags);
   XF_HIP(hipDeviceSynchronize());
   uploaded = true;
@@ -1833,6 +2018,7 @@ void Engine::set_tiling(int ty, int chunks_x, int flags) {
   plan.tile_y = ty;
   plan.chunks_x = chunks_x;
   plan.tiling_flags = flags;
+  step3_auto = ty == 0 && chunks_x == 0 && !(flags & XF_TILE_SET);
   // 64 x tile_y threads must fit the kernels' __launch_bounds__(256)
   tile_y = ty > 0 ? std::min(ty, 4) : 1;
   if (flags & XF_TILE_SET) {
@@ -1872,11 +2058,7 @@ void Engine::set_tiling(int ty, int chunks_x, int flags) {
     chunk = static_cast<int>((nx + 1 + nch - 1) / nch);
     nch_eff = static_cast<int>((nx + 1 + chunk - 1) / chunk);
   }
-  if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
-  if (graph) (void)hipGraphDestroy(graph);
-  graph_exec = nullptr;
-  graph = nullptr;
-  graph_ready = false;
+  drop_graph();
   if (pml_streams && dim == 3 && stream && build_tile_lists() != XF_OK) pml_streams = 0;
   layout_desc = std::string("dim=") + std::to_string(dim) + " pad_stride=" + std::to_string(dim == 3 ? sy : sx) +
                 " id_bytes=" + std::to_string(id_bytes) + " coeff=" + (dense ? "dense" : "table") +
@@ -1888,7 +2070,10 @@ void Engine::set_tiling(int ty, int chunks_x, int flags) {
                 " klanes=" + std::to_string(klanes) + " pml_streams=" + std::to_string(pml_streams) +
                 " pml_faces=" + std::to_string(pml.size()) + " cpsi_tab=" + std::to_string(cpsi_matched()) +
                 " ade_cells=" + std::to_string(ade_cells.size()) +
-                (has_ade ? " ade_rows=" + std::to_string(ade_rows) : std::string());
+                (has_ade ? " ade_rows=" + std::to_string(ade_rows) : std::string()) +
+                " step3=" + std::to_string(use_step3() ? 1 : 0) +
+                (use_step3() ? " step3_chunk=" + std::to_string(step3_chunk) + " step3_rows=" + std::to_string(step3_rows)
+                             : std::string());
 }
 
 int Engine::snapshot() {
@@ -1899,7 +2084,7 @@ int Engine::snapshot() {
     for (size_t q = 0; q < state.size(); ++q) XF_TRY(alloc(&backup[q], state[q].second));
   }
   for (size_t q = 0; q < state.size(); ++q)
-    XF_HIP(hipMemcpyAsync(backup[q], state[q].first, state[q].second, hipMemcpyDeviceToDevice, stream));
+    XF_HIP(hipMemcpyAsync(backup[q], live(state[q].first), state[q].second, hipMemcpyDeviceToDevice, stream));
   XF_HIP(hipStreamSynchronize(stream));
   lb_rec_count_saved = lb_rec_count;
   return XF_OK;
@@ -1909,7 +2094,7 @@ int Engine::restore() {
   if (backup.size() != state.size()) return fail(XF_ERR_STATE, "restore without snapshot");
   XF_HIP(hipSetDevice(device));
   for (size_t q = 0; q < state.size(); ++q)
-    XF_HIP(hipMemcpyAsync(state[q].first, backup[q], state[q].second, hipMemcpyDeviceToDevice, stream));
+    XF_HIP(hipMemcpyAsync(live(state[q].first), backup[q], state[q].second, hipMemcpyDeviceToDevice, stream));
   XF_HIP(hipStreamSynchronize(stream));
   lb_rec_count = lb_rec_count_saved;
   return XF_OK;
@@ -2533,15 +2718,7 @@ int Engine::launch_e(int t, const int* tp) {
 #undef XF_LE3D
     XF_HIP(hipGetLastError());
     if (split_z()) XF_TRY(launch_pml_z<S>(true, stream));
-    if (has_ade && ade.n > 0) {
-      dim3 b1(256), g1((unsigned)((ade.n + 255) / 256));
-      if (id_bytes == 1)
-        hipLaunchKernelGGL((k_ade_e3<S, uint8_t>), g1, b1, 0, stream, f, static_cast<const uint8_t*>(eid), tab, ade, d, scl,
-                           dense9<C>(true));
-      else
-        hipLaunchKernelGGL((k_ade_e3<S, uint16_t>), g1, b1, 0, stream, f, static_cast<const uint16_t*>(eid), tab, ade, d, scl,
-                           dense9<C>(true));
-    }
+    XF_TRY(launch_ade<S>(stream));
   } else {
     dim3 block(64, 4);
     dim3 grid((unsigned)((ny + 1 + 63) / 64), (unsigned)((nx + 1 + 3) / 4));
@@ -2564,6 +2741,161 @@ int Engine::launch_e(int t, const int* tp) {
 }
 
 
+// The dispersive cells' E update, after the pass that left them alone.
+template <typename S>
+int Engine::launch_ade(hipStream_t st) {
+  using C = typename Store<S>::C;
+  if (!has_ade || ade.n <= 0) return XF_OK;
+  const dim3 block(256), grid((unsigned)((ade.n + 255) / 256));
+  const C* tab = static_cast<const C*>(etab);
+  if (id_bytes == 1)
+    hipLaunchKernelGGL((k_ade_e3<S, uint8_t>), grid, block, 0, st, make_fields<S>(*this), static_cast<const uint8_t*>(eid),
+                       tab, ade, make_dims(*this), make_scales<C>(*this), dense9<C>(true));
+  else
+    hipLaunchKernelGGL((k_ade_e3<S, uint16_t>), grid, block, 0, st, make_fields<S>(*this), static_cast<const uint16_t*>(eid),
+                       tab, ade, make_dims(*this), make_scales<C>(*this), dense9<C>(true));
+  XF_HIP(hipGetLastError());
+  return XF_OK;
+}
+
+// k_step3's descriptor of a step from the current set into the other.
+template <typename S>
+Step3Pass<S> Engine::step3_pass() const {
+  using C = typename Store<S>::C;
+  Step3Pass<S> D{};
+  for (int c = 0; c < 3; ++c) {
+    D.e[c] = static_cast<const S*>(fld[c]);
+    D.h[c] = static_cast<const S*>(fld[3 + c]);
+    D.eo[c] = static_cast<S*>(fld2[c]);
+    D.ho[c] = static_cast<S*>(fld2[3 + c]);
+  }
+  D.ids = static_cast<const uint8_t*>(step3_ids);
+  D.tab = static_cast<const C*>(step3_tab);
+  D.ntab = step3_rows;
+  D.ade = has_ade ? 1 : 0;
+  D.dmask = step3_dmask;
+  D.d = make_dims(*this);
+  D.sc = make_scales<C>(*this);
+  D.nkb = static_cast<int>((nz + 64) / 64);
+  D.njb = static_cast<int>((ny + kStep3Rows) / kStep3Rows);
+  D.chunk = step3_chunk;
+  D.nch = static_cast<int>((nx + step3_chunk) / step3_chunk);
+  PmlPass<C> ph{}, pe{};
+  fill_pml_pass<C>(*this, ph, false);
+  fill_pml_pass<C>(*this, pe, true);
+  D.n_face = ph.n;
+  std::vector<int> order(static_cast<size_t>(ph.n));
+  std::iota(order.begin(), order.end(), 0);
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+    return std::make_pair(ph.f[a].axis, ph.f[a].c0) < std::make_pair(ph.f[b].axis, ph.f[b].c0);
+  });
+  for (int n = 0; n < D.n_face; ++n) {
+    const int q = order[static_cast<size_t>(n)];
+    D.face[0][n] = step3_face<C>(ph.f[q], false, static_cast<C*>(pml[q].psi2[0]), static_cast<C*>(pml[q].psi2[1]));
+    D.face[1][n] = step3_face<C>(pe.f[q], true, pe.f[q].psi_a, pe.f[q].psi_b);
+  }
+  if (sc->tfsf) {
+    TfsfPass<C> T[2]{};
+    fill_tfsf_pass<C>(*this, T[0], 0);
+    fill_tfsf_pass<C>(*this, T[1], 1);
+    const xf_array* proj[3] = {&sc->tfsf->proj_x_int, &sc->tfsf->proj_y_int, &sc->tfsf->proj_z_int};
+    for (int d = 0; d < 3; ++d) {
+      D.proj_int[d] = T[0].proj_int[d];
+      D.proj_half[d] = T[0].proj_half[d];
+      D.g[d] = T[0].g[d];
+      D.n_proj[d] = static_cast<int>(proj[d]->shape[0]);
+    }
+    for (int p = 0; p < 2; ++p) {
+      D.inc[p] = T[p].inc;
+      D.n_aux[p] = T[p].n_aux;
+      D.n_job[p] = p == 1 && has_ade ? 0 : T[p].njob;  // a dispersive cell takes them after its ADE update
+      for (int q = 0; q < D.n_job[p]; ++q) D.job[p][q] = step3_job<C>(T[p].job[q], T[p]);
+    }
+  }
+  return D;
+}
+
+// Whether k_step3 holds the CPML as it is: faces across one axis so far apart
+// that no node meets two, no plane and its successor two x faces and no block
+// two y faces; and psi arrays that 32-bit byte offsets reach, in rows that 24
+// bits count.
+bool Engine::step3_faces() const {
+  const int gap[3] = {1, kStep3Rows + 2, 0};
+  for (int pass = 0; pass < 2; ++pass) {
+    PmlPass<double> P{};
+    fill_pml_pass<double>(*this, P, pass == 1);
+    for (int q = 0; q < P.n; ++q) {
+      const PmlFace<double>& F = P.f[q];
+      for (int n = 0; n < q; ++n)
+        if (P.f[n].axis == F.axis && P.f[n].c0 < F.c1 + gap[F.axis] && F.c0 < P.f[n].c1 + gap[F.axis]) return false;
+      const xf_pml& S = sc->pml[pml_order[static_cast<size_t>(q)]];
+      for (const xf_array* psi : {&S.ea_psi_hb, &S.eb_psi_ha, &S.ha_psi_eb, &S.hb_psi_ea})
+        if (numel(*psi) >= (int64_t(1) << 28)) return false;
+      if (std::max(F.sa2, F.sb2) >= (1 << 24) || ny >= (1 << 24)) return false;
+    }
+  }
+  return true;
+}
+
+// Planes per chunk of k_step3 for the grids that share a launch.  A block
+// takes about chunk + 3 plane times (its prologue, and its first plane's H
+// formed twice), and the launch as many rounds of blocks as do not fit the
+// device at once: the chunk with the least rounds * (chunk + 3), which gives
+// one round of long marches to a mid-sized grid and short marches to a small one.
+template <typename S>
+int step3_pick_chunk(const std::vector<const Engine*>& grids, bool pml, size_t lds) {
+  int cus = 0;
+  if (grids.empty() || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, grids[0]->device) != hipSuccess)
+    cus = 256;
+  const int64_t slots = static_cast<int64_t>(std::max(1, cus)) * step3_blocks_per_cu<S>(pml, lds);
+  int best = 2;
+  int64_t least = INT64_MAX;
+  for (int chunk = 2; chunk <= kStep3MaxChunk; ++chunk) {
+    int64_t blocks = 0;
+    for (const Engine* E : grids)
+      blocks += ((E->nz + 64) / 64) * ((E->ny + kStep3Rows) / kStep3Rows) * ((E->nx + chunk) / chunk);
+    const int64_t cost = (blocks + slots - 1) / slots * (chunk + 3);
+    if (cost < least) {
+      least = cost;
+      best = chunk;
+    }
+  }
+  return best;
+}
+
+template <typename S>
+int Engine::step3_describe() {
+  step3_chunk = step3_pick_chunk<S>({this}, !pml.empty(), step3_lds());
+  Step3Pass<S> D[2];
+  D[0] = step3_pass<S>();
+  step3_swap();
+  D[1] = step3_pass<S>();
+  step3_swap();
+  const int64_t blocks = static_cast<int64_t>(D[0].nkb) * D[0].njb * D[0].nch;
+  if (blocks > INT_MAX / 2) {
+    step3_ready = false;
+    return XF_OK;
+  }
+  step3_blocks = static_cast<int>(blocks);
+  XF_TRY(alloc(&step3_desc, sizeof(D)));
+  XF_HIP(hipMemcpy(step3_desc, D, sizeof(D), hipMemcpyHostToDevice));
+  const int start[2] = {0, step3_blocks};
+  void* p = nullptr;
+  XF_TRY(alloc(&p, sizeof(start)));
+  step3_start = static_cast<int*>(p);
+  XF_HIP(hipMemcpy(step3_start, start, sizeof(start), hipMemcpyHostToDevice));
+  return XF_OK;
+}
+
+// One step from the current set into the other, which becomes current.
+template <typename S>
+int Engine::launch_step3(int t, const int* tp) {
+  XF_HIP(step3_launch<S>(static_cast<const Step3Pass<S>*>(step3_desc) + step3_set, step3_start, 1, step3_blocks,
+                         !pml.empty(), step3_lds(), t, tp, stream));
+  step3_swap();
+  return launch_ade<S>(stream);
+}
+
 template <typename S>
 int Engine::launch_post_h(int t, const int* tp) {
   using C = typename Store<S>::C;
@@ -2581,9 +2913,10 @@ int Engine::launch_post_h(int t, const int* tp) {
 template <typename S>
 int Engine::launch_post_e(int t, const int* tp) {
   using C = typename Store<S>::C;
-  if (sc->tfsf && !tfsf_fused()) {
+  // the one-pass step has applied them, unless ADE cells were still to update
+  if (sc->tfsf && !tfsf_fused() && !(use_step3() && !has_ade)) {
     TfsfPass<C> P{};
-    fill_tfsf_pass<C>(*this, P, 1, tfsf_ztail());
+    fill_tfsf_pass<C>(*this, P, 1, !use_step3() && tfsf_ztail());
     if (P.total > 0)
       hipLaunchKernelGGL((k_tfsf<S>), dim3((unsigned)((P.total + 255) / 256)), dim3(256), 0, stream,
                          make_fields<S>(*this), P, t, tp, make_scales<C>(*this), make_dims(*this), dim == 2 ? 1 : 0);
@@ -2673,11 +3006,14 @@ template <typename S>
 int Engine::launch_step(int t, bool use_tdev, bool timing_events, hipEvent_t* ev) {
   const int* tp = use_tdev ? t_dev : nullptr;
   if (timing_events) XF_HIP(hipEventRecord(ev[0], stream));
-  XF_TRY(launch_h<S>(t, tp));
+  if (!use_step3()) XF_TRY(launch_h<S>(t, tp));
   if (timing_events) XF_HIP(hipEventRecord(ev[1], stream));
-  XF_TRY(launch_post_h<S>(t, tp));
+  if (!use_step3()) XF_TRY(launch_post_h<S>(t, tp));
   if (timing_events) XF_HIP(hipEventRecord(ev[2], stream));
-  XF_TRY(launch_e<S>(t, tp));
+  if (use_step3())
+    XF_TRY(launch_step3<S>(t, tp));
+  else
+    XF_TRY(launch_e<S>(t, tp));
   if (timing_events) XF_HIP(hipEventRecord(ev[3], stream));
   XF_TRY(launch_post_e<S>(t, tp));
   if (timing_events) XF_HIP(hipEventRecord(ev[4], stream));
@@ -2732,26 +3068,43 @@ int Engine::run(int64_t n) {
   };
   if (graph_on && !timing_on) {
     if (!graph_ready) {
-      XF_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-      int st;
-      switch (plan.precision) {
-        case XF_FP64:
-          st = launch_step<double>(0, true, false, nullptr);
-          break;
-        case XF_FP32:
-          st = launch_step<float>(0, true, false, nullptr);
-          break;
-        case XF_BF16_COMP:
-          st = launch_step<Bf16c>(0, true, false, nullptr);
-          break;
-        case XF_FP16_STORE:
-          st = launch_step<__half>(0, true, false, nullptr);
-          break;
-        default:
-          st = launch_step<__hip_bfloat16>(0, true, false, nullptr);
+      drop_graph();
+      const int set0 = step3_set;
+      // a one-pass step leaves the fields in the other set, so the steps from
+      // the two sets are two graphs; capturing both leaves the sets as they were
+      const int n_graph = use_step3() ? 2 : 1;
+      for (int q = 0; q < n_graph; ++q) {
+        const int slot = use_step3() ? step3_set : 0;
+        XF_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+        int st;
+        switch (plan.precision) {
+          case XF_FP64:
+            st = launch_step<double>(0, true, false, nullptr);
+            break;
+          case XF_FP32:
+            st = launch_step<float>(0, true, false, nullptr);
+            break;
+          case XF_BF16_COMP:
+            st = launch_step<Bf16c>(0, true, false, nullptr);
+            break;
+          case XF_FP16_STORE:
+            st = launch_step<__half>(0, true, false, nullptr);
+            break;
+          default:
+            st = launch_step<__hip_bfloat16>(0, true, false, nullptr);
+        }
+        const int ended = end_capture(stream, st, &graph[slot]);
+        if (ended != XF_OK) {
+          // the captured steps did not run: back to the set the fields are in
+          if (use_step3() && step3_set != set0) step3_swap();
+          return ended;
+        }
+        const hipError_t made = hipGraphInstantiate(&graph_exec[slot], graph[slot], nullptr, nullptr, 0);
+        if (made != hipSuccess) {
+          if (use_step3() && step3_set != set0) step3_swap();
+          return fail(XF_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(made));
+        }
       }
-      XF_TRY(end_capture(stream, st, &graph));
-      XF_HIP(hipGraphInstantiate(&graph_exec, graph, nullptr, nullptr, 0));
       graph_ready = true;
     }
     const int t0 = static_cast<int>(cur_step);
@@ -2759,7 +3112,8 @@ int Engine::run(int64_t n) {
     XF_HIP(hipStreamSynchronize(stream));
     XF_HIP(hipEventRecord(run0, stream));
     for (int64_t s = 0; s < n; ++s) {
-      XF_HIP(hipGraphLaunch(graph_exec, stream));
+      XF_HIP(hipGraphLaunch(graph_exec[use_step3() ? step3_set : 0], stream));
+      if (use_step3()) step3_swap();
       if (wd && ((cur_step + s + 1) % wd == 0 || s + 1 == n)) XF_TRY(watch(s + 1));
     }
   } else {
@@ -2794,7 +3148,7 @@ int Engine::run(int64_t n) {
     timing.yee_h_launches += n;
     timing.yee_e_launches += n;
   }
-  timing.bytes_per_cell_step = bytes_per_cell_step();
+  timing.bytes_per_cell_step = bytes_per_cell_step(use_step3());
   cur_step += n;
   if (has_lb && lbd.mode == XF_LB_RECORD) lb_rec_count = lb_recorded_after(cur_step);
   if (first_bad != 0xffffffffu)
@@ -2892,7 +3246,7 @@ int xf_get_timing(const xf_handle* h, xf_timing* out) {
   return xf::guarded([&]() -> int {
     if (!h || !out) return xf::fail(XF_ERR_INVALID, "null argument");
     *out = h->eng.timing;
-    out->bytes_per_cell_step = h->eng.bytes_per_cell_step();
+    out->bytes_per_cell_step = h->eng.bytes_per_cell_step(h->eng.use_step3());
     return XF_OK;
   });
 }

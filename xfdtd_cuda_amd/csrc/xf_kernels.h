@@ -545,6 +545,197 @@ struct LbItem {
   LbDev L;
 };
 
+// One step of one grid in a single pass over memory (k_step3): both passes'
+// tables, CPML faces and TF/SF jobs, and the two sets of fields and H-pass
+// psi it goes between.  In device memory, one per grid and direction.
+constexpr int kStep3Rows = 6;       // j-rows a block owns
+constexpr int kStep3MaxRows = 256;  // coefficient rows (pairs of E and H rows) the block's table holds (one-byte ids)
+constexpr int kStep3AdeRows = 64;   // ... with dispersive media, whose rows are a 64-bit mask
+constexpr int kStep3MaxChunk = 32;  // planes a block marches through at most
+constexpr int kStep3Proj = 72;      // projections of one axis a block holds: its 64 lanes (or 33 planes, or rows) and 2 a side
+constexpr int kStep3Inc = 192;      // incident values of one table row a block holds
+constexpr int kStep3ZJobs = 4;      // TF/SF jobs of z faces a block works out before it marches, a pass
+
+// What a plane's correction by a CPML face of one pass takes, in one scalar
+// load.  psi of node (i, j, k) is at i * plane + j * row + k past the biased
+// pointer (pml_face's layouts for all three axes); psi_a corrects the planes
+// [lo, hi_a), psi_b [lo, hi_b).
+typedef int step3_i16 __attribute__((vector_size(64)));
+template <typename C>
+struct alignas(64) Step3Face {
+  const C* a;  // psi_a, psi_b read
+  const C* b;
+  C* oa;  // ... and written (the H pass: the other set's)
+  C* ob;
+  uint32_t plane_a, plane_b;  // bytes
+  int row_a, row_b;           // values
+  int lo, hi_a, hi_b;
+  int t_ab;  // PmlFace::ta and tb, a byte each (0xff: none)
+  // (a second line) c_psi, indexed like psi, where it is no table row; PmlFace's
+  // ranges; a profile value is at node + off
+  const C* cpa;
+  const C* cpb;
+  int axis, c0, c1, a0, a1, b0, b1, off;
+  const C* ca;
+  const C* cb;
+};
+
+// A TF/SF job: its box, and where the projections of a node that its
+// incident value takes are among the block's (kStep3Proj per axis and grid).
+template <typename C>
+struct alignas(64) Step3Job {
+  int lo[3], hi[3];
+  int at[3];
+  int comp;
+  int axis;
+  C coef, tr;
+};
+
+// step3_face, step3_job: from the two-pass kernels' descriptors.
+template <typename C>
+Step3Face<C> step3_face(const PmlFace<C>& F, bool is_e, C* oa, C* ob) {
+  Step3Face<C> D{};
+  const int64_t sa = F.sa1 * F.sa2, sb = F.sb1 * F.sb2;
+  const int64_t ka = F.nstart * (F.axis == 0 ? sa : F.axis == 1 ? F.sa2 : 1);
+  const int64_t kb = F.nstart * (F.axis == 0 ? sb : F.axis == 1 ? F.sb2 : 1);
+  D.a = F.psi_a - ka;
+  D.b = F.psi_b - kb;
+  D.oa = oa - ka;
+  D.ob = ob - kb;
+  D.cpa = F.cpsi_a - ka;
+  D.cpb = F.cpsi_b - kb;
+  D.plane_a = static_cast<uint32_t>(sa * sizeof(C));
+  D.plane_b = static_cast<uint32_t>(sb * sizeof(C));
+  D.row_a = static_cast<int>(F.sa2);
+  D.row_b = static_cast<int>(F.sb2);
+  D.t_ab = (F.ta & 0xff) | (F.tb & 0xff) << 8;
+  D.axis = F.axis;
+  D.c0 = F.c0;
+  D.c1 = F.c1;
+  D.a0 = F.a0;
+  D.a1 = F.a1;
+  D.b0 = F.b0;
+  D.b1 = F.b1;
+  D.off = F.off_c - F.gstart;
+  D.ca = F.ca;
+  D.cb = F.cb;
+  // planes: the main range of an x face; else the lateral range that holds i,
+  // which one of the two psi takes closed and the other half-open
+  D.lo = F.axis == 0 ? F.c0 : F.axis == 1 ? F.b0 : F.a0;
+  const int hi = F.axis == 0 ? F.c1 : F.axis == 1 ? F.b1 : F.a1;
+  const bool a_closed = (F.axis == 1) == is_e;
+  D.hi_a = F.axis == 0 ? hi : a_closed ? hi + 1 : hi;
+  D.hi_b = F.axis == 0 ? hi : a_closed ? hi : hi + 1;
+  return D;
+}
+template <typename C>
+Step3Job<C> step3_job(const TfsfJob<C>& J, const TfsfPass<C>& T) {
+  Step3Job<C> D{};
+  const bool is_e = T.is_e != 0;
+  const int axis = J.face >> 1, a = axis == 2 ? 0 : axis + 1;
+  const int dual = J.comp == a ? (a == 2 ? 0 : a + 1) : a;
+  const int back = (J.face & 1) ? 0 : is_e ? -1 : 1;
+  for (int d = 0; d < 3; ++d) {
+    D.lo[d] = J.o[d];
+    D.hi[d] = J.o[d] + J.n[d];
+    // incident E (H pass) is on the half grid along its own axis only,
+    // incident H across it
+    const int half = (dual == d) != is_e ? 1 : 0;
+    D.at[d] = (2 * d + half) * kStep3Proj + 2 + (axis == d ? back : 0);
+  }
+  D.comp = J.comp;
+  D.axis = axis;
+  D.coef = J.coef;
+  D.tr = T.tr[dual];
+  return D;
+}
+
+template <typename S>
+struct Step3Pass {
+  using C = typename Store<S>::C;
+  const S* e[3];
+  const S* h[3];
+  S* eo[3];
+  S* ho[3];
+  const uint8_t* ids;    // per node (padded layout): row of tab, 0 where the node is no cell
+  const C* tab;          // 18 coefficients a row: the E pass's nine, the H pass's nine
+  int ntab;
+  int ade;               // rows of dmask are left to the ADE kernel
+  uint64_t dmask;
+  Dims d;
+  Scales<C> sc;
+  int nkb, njb, nch, chunk;
+  int n_face;
+  Step3Face<C> face[2][kMaxPml];  // of the H and the E pass, by axis, then by place
+  int n_job[2];                   // TF/SF jobs of the H and the E pass
+  Step3Job<C> job[2][kMaxTfsfJobs];
+  const C* proj_int[3];
+  const C* proj_half[3];
+  int g[3];
+  const C* inc[2];  // e_inc and h_inc, and their row lengths
+  int64_t n_aux[2];
+  int n_proj[3];         // lengths of the projection arrays
+};
+
+// Launches k_step3 over `blocks` blocks: grid g owns the blocks
+// [block_start[g], block_start[g + 1]).  lds: bytes of the largest table.
+template <typename S>
+hipError_t step3_launch(const Step3Pass<S>* passes, const int* block_start, int n, int blocks, bool pml, size_t lds,
+                        int t_arg, const int* t_dev, hipStream_t stream);
+
+// Blocks of k_step3 one CU holds at a time.
+template <typename S>
+int step3_blocks_per_cu(bool pml, size_t lds);
+
+// Faces of the pass whose corrected box the column (j, k) can meet for some
+// i in [i0, i1): a superset of what pml_face accepts (lateral ranges taken
+// with their one-node extension).  Worked out once per tile, it lets the
+// interior columns skip the CPML code of every plane.
+template <typename C>
+__device__ __forceinline__ unsigned pml_mask(const PmlPass<C>& P, int i0, int i1, int j, int k) {
+  unsigned bits = 0;
+  for (int q = 0; q < P.n; ++q) {
+    const PmlFace<C>& F = P.f[q];
+    bool hit;
+    if (F.axis == 0)  // c = i, a = j, b = k
+      hit = F.c0 < i1 && F.c1 > i0 && j >= F.a0 && j <= F.a1 && k >= F.b0 && k <= F.b1;
+    else if (F.axis == 1)  // c = j, a = k, b = i
+      hit = j >= F.c0 && j < F.c1 && k >= F.a0 && k <= F.a1 && F.b0 < i1 && F.b1 >= i0;
+    else  // c = k, a = i, b = j
+      hit = k >= F.c0 && k < F.c1 && F.a0 < i1 && F.a1 >= i0 && j >= F.b0 && j <= F.b1;
+    if (hit) bits |= 1u << q;
+  }
+  return bits;
+}
+
+// exInc..hzInc (tfsf_corrector.cu:18-130): interpolated 1-D incident value.
+// P is a TfsfPass or a TfsfZTail (the same field names).
+template <template <typename> class Pass, typename C>
+__device__ __forceinline__ C tfsf_inc(const Pass<C>& P, bool inc_is_e, int comp, int t,
+                                      int i, int j, int k) {
+  const int li = i - P.g[0], lj = j - P.g[1], lk = k - P.g[2];
+  C proj;
+  if (inc_is_e) {
+    if (comp == 0)
+      proj = gp(P.proj_half[0])[li + 1] + gp(P.proj_int[1])[lj] + gp(P.proj_int[2])[lk];
+    else if (comp == 1)
+      proj = gp(P.proj_int[0])[li] + gp(P.proj_half[1])[lj + 1] + gp(P.proj_int[2])[lk];
+    else
+      proj = gp(P.proj_int[0])[li] + gp(P.proj_int[1])[lj] + gp(P.proj_half[2])[lk + 1];
+  } else {
+    if (comp == 0)
+      proj = gp(P.proj_int[0])[li] + gp(P.proj_half[1])[lj + 1] + gp(P.proj_half[2])[lk + 1] - (C)0.5;
+    else if (comp == 1)
+      proj = gp(P.proj_half[0])[li + 1] + gp(P.proj_int[1])[lj] + gp(P.proj_half[2])[lk + 1] - (C)0.5;
+    else
+      proj = gp(P.proj_half[0])[li + 1] + gp(P.proj_half[1])[lj + 1] + gp(P.proj_int[2])[lk] - (C)0.5;
+  }
+  const uint64_t index = (uint64_t)proj;
+  const C weight = proj - (C)index;
+  const __attribute__((address_space(1))) C* row = gp(P.inc) + (int64_t)t * P.n_aux;
+  return P.tr[comp] * ((1 - weight) * row[index] + weight * row[index + 1]);
+}
+
 }  // namespace xf
 
 #endif  // XF_KERNELS_H_

@@ -184,34 +184,6 @@ __device__ __forceinline__ const C* load_table(const C* __restrict__ g, int nval
 }
 
 // ------------------------------------------------------------------ TFSF
-// exInc..hzInc (tfsf_corrector.cu:18-130): interpolated 1-D incident value.
-// P is a TfsfPass or a TfsfZTail (the same field names).
-template <template <typename> class Pass, typename C>
-__device__ __forceinline__ C tfsf_inc(const Pass<C>& P, bool inc_is_e, int comp, int t,
-                                      int i, int j, int k) {
-  const int li = i - P.g[0], lj = j - P.g[1], lk = k - P.g[2];
-  C proj;
-  if (inc_is_e) {
-    if (comp == 0)
-      proj = gp(P.proj_half[0])[li + 1] + gp(P.proj_int[1])[lj] + gp(P.proj_int[2])[lk];
-    else if (comp == 1)
-      proj = gp(P.proj_int[0])[li] + gp(P.proj_half[1])[lj + 1] + gp(P.proj_int[2])[lk];
-    else
-      proj = gp(P.proj_int[0])[li] + gp(P.proj_int[1])[lj] + gp(P.proj_half[2])[lk + 1];
-  } else {
-    if (comp == 0)
-      proj = gp(P.proj_int[0])[li] + gp(P.proj_half[1])[lj + 1] + gp(P.proj_half[2])[lk + 1] - (C)0.5;
-    else if (comp == 1)
-      proj = gp(P.proj_half[0])[li + 1] + gp(P.proj_int[1])[lj] + gp(P.proj_half[2])[lk + 1] - (C)0.5;
-    else
-      proj = gp(P.proj_half[0])[li + 1] + gp(P.proj_half[1])[lj + 1] + gp(P.proj_int[2])[lk] - (C)0.5;
-  }
-  const uint64_t index = (uint64_t)proj;
-  const C weight = proj - (C)index;
-  const __attribute__((address_space(1))) C* row = gp(P.inc) + (int64_t)t * P.n_aux;
-  return P.tr[comp] * ((1 - weight) * row[index] + weight * row[index + 1]);
-}
-
 #include "xf_yee3d.inl"
 
 // All TFSF face corrections of one pass in one launch.  Each thread owns a

@@ -85,27 +85,6 @@ __device__ __forceinline__ void st3(S* const* dst, int64_t idx, const typename S
   }
 }
 
-// Faces of the pass whose corrected box the column (j, k) can meet for some
-// i in [i0, i1): a superset of what pml_face accepts (lateral ranges taken
-// with their one-node extension).  Worked out once per tile, it lets the
-// interior columns skip the CPML code of every plane.
-template <typename C>
-__device__ __forceinline__ unsigned pml_mask(const PmlPass<C>& P, int i0, int i1, int j, int k) {
-  unsigned bits = 0;
-  for (int q = 0; q < P.n; ++q) {
-    const PmlFace<C>& F = P.f[q];
-    bool hit;
-    if (F.axis == 0)  // c = i, a = j, b = k
-      hit = F.c0 < i1 && F.c1 > i0 && j >= F.a0 && j <= F.a1 && k >= F.b0 && k <= F.b1;
-    else if (F.axis == 1)  // c = j, a = k, b = i
-      hit = j >= F.c0 && j < F.c1 && k >= F.a0 && k <= F.a1 && F.b0 < i1 && F.b1 >= i0;
-    else  // c = k, a = i, b = j
-      hit = k >= F.c0 && k < F.c1 && F.a0 < i1 && F.a1 >= i0 && j >= F.b0 && j <= F.b1;
-    if (hit) bits |= 1u << q;
-  }
-  return bits;
-}
-
 // The z-face CPML corrections of the tile's column (j, k) over [i0, i1),
 // applied after its march (XF_TILE_PML_ZTAIL): the lanes whose column lies
 // in a z slab revisit their nodes, which this lane stored itself, so the
