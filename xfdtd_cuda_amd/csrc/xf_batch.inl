@@ -718,7 +718,21 @@ int Batch::run(int64_t n) {
 int Batch::download() {
   if (!uploaded) return fail(XF_ERR_STATE, "download before upload");
   XF_HIP(hipStreamSynchronize(stream));
-  for (auto& h : inst) XF_TRY(h->eng.download());
+  if (inst.empty()) return XF_OK;
+  // one pass through the staging slots for every grid
+  size_t most = 0, all = 0;
+  for (auto& h : inst) {
+    XF_HIP(hipStreamSynchronize(h->eng.stream));
+    most = std::max(most, h->eng.plane_bytes());
+    all += h->eng.drain_bytes();
+  }
+  {
+    Drain out(inst[0]->eng.stages, stream, most, all);
+    XF_HIP(out.open());
+    for (auto& h : inst) XF_TRY(h->eng.drain(out));
+    XF_HIP(out.finish());
+  }
+  for (auto& h : inst) XF_TRY(h->eng.download_rest());
   return XF_OK;
 }
 

@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "../../include/xfdtd_hip.h"
+#include "xf_drain.h"
 #include "xf_kernels.inl"
 
 namespace xf {
@@ -391,17 +392,6 @@ struct Engine {
     return upload_vec(p, v);
   }
 
-  int download_c(double* dst, const void* p, int64_t n) {
-    if (plan.precision == XF_FP64) {
-      XF_HIP(hipMemcpy(dst, p, n * sizeof(double), hipMemcpyDeviceToHost));
-      return XF_OK;
-    }
-    std::vector<float> v(n);
-    XF_HIP(hipMemcpy(v.data(), p, n * sizeof(float), hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < n; ++i) dst[i] = v[i];
-    return XF_OK;
-  }
-
   int validate();
   int build_tfsf_jobs();
   int check_overlaps();
@@ -409,7 +399,13 @@ struct Engine {
   bool dispersive(int64_t i, int64_t j, int64_t k) const;
   int upload();
   int pack_fields();
-  int unpack_fields();
+  int unpack_fields(Drain& out);
+  int drain_c(Drain& out, double* dst, const void* p, int64_t n);
+  int drain(Drain& out);
+  size_t plane_bytes() const { return static_cast<size_t>(sx) * esize; }
+  size_t drain_bytes() const;
+  int download_rest();
+  std::shared_ptr<StagePool> stages{StagePool::shared()};
   int build_ids();
   int upload_pml();
   int upload_tfsf();
@@ -1081,37 +1077,51 @@ int Engine::pack_fields() {
   return XF_OK;
 }
 
-int Engine::unpack_fields() {
+// Device arrays on their way to the host: read into pinned slots by turns, a
+// slot filled while the host's threads convert the other into the caller's
+// arrays.
+int Engine::unpack_fields(Drain& out) {
   xf_array* dst[6] = {&sc->ex, &sc->ey, &sc->ez, &sc->hx, &sc->hy, &sc->hz};
   const int prec = plan.precision;
   const double sh = (prec == XF_BF16_STORE || prec == XF_BF16_COMP || prec == XF_FP16_STORE) ? 376.730313668 : 1.0;
-  std::vector<unsigned char> buf(total * esize);
+  const size_t plane = static_cast<size_t>(sx) * esize;  // compensated bf16: whole 64-value blocks
   for (int c = 0; c < 6; ++c) {
     if (!fld[c]) continue;
-    XF_HIP(hipMemcpy(buf.data(), fld[c], total * esize, hipMemcpyDeviceToHost));
-    xf_array& a = *dst[c];
+    const xf_array& a = *dst[c];
     const double inv = c < 3 ? 1.0 : 1.0 / sh;
-    host_parallel_for(a.shape[0], [&](int64_t i0, int64_t i1) {
-    for (int64_t i = i0; i < i1; ++i)
-      for (int64_t j = 0; j < a.shape[1]; ++j)
-        for (int64_t k = 0; k < a.shape[2]; ++k) {
-          const int64_t idx = dim == 3 ? i * sx + j * sy + k : i * sx + j;
-          double v;
+    const int64_t nj = a.shape[1], nk = a.shape[2], step = std::max<int64_t>(1, static_cast<int64_t>(out.slot_bytes() / plane));
+    for (int64_t p0 = 0; p0 < a.shape[0]; p0 += step) {
+      const int64_t planes = std::min(step, a.shape[0] - p0);
+      double* to = a.data + p0 * nj * nk;
+      // rows [lo, hi) of these planes
+      auto put = [=, this](const unsigned char* from, int64_t lo, int64_t hi) {
+        for (int64_t r = lo; r < hi; ++r) {
+          const int64_t at = dim == 3 ? r / nj * sx + r % nj * sy : r / nj * sx + r % nj;
+          double* const o = to + r * nk;
+          // a 2-D grid has one value of k
+          const int64_t n = dim == 3 ? nk : 1;
           if (prec == XF_FP64)
-            v = reinterpret_cast<const double*>(buf.data())[idx];
+            std::memcpy(o, reinterpret_cast<const double*>(from) + at, static_cast<size_t>(n) * sizeof(double));
           else if (prec == XF_FP32)
-            v = reinterpret_cast<const float*>(buf.data())[idx];
-          else if (prec == XF_BF16_COMP) {
-            const unsigned char* b = buf.data() + (idx >> 6) * 192;
-            v = static_cast<double>(bf16c_decode(reinterpret_cast<const uint16_t*>(b)[idx & 63],
-                                                 reinterpret_cast<const int8_t*>(b + 128)[idx & 63])) * inv;
-          } else if (prec == XF_FP16_STORE)
-            v = static_cast<double>(__half2float(reinterpret_cast<const __half*>(buf.data())[idx])) * inv;
+            for (int64_t k = 0; k < n; ++k) o[k] = reinterpret_cast<const float*>(from)[at + k];
+          else if (prec == XF_BF16_COMP)
+            for (int64_t k = 0; k < n; ++k) {
+              const unsigned char* b = from + ((at + k) >> 6) * 192;
+              o[k] = static_cast<double>(bf16c_decode(reinterpret_cast<const uint16_t*>(b)[(at + k) & 63],
+                                                      reinterpret_cast<const int8_t*>(b + 128)[(at + k) & 63])) * inv;
+            }
+          else if (prec == XF_FP16_STORE)
+            for (int64_t k = 0; k < n; ++k)
+              o[k] = static_cast<double>(__half2float(reinterpret_cast<const __half*>(from)[at + k])) * inv;
           else
-            v = static_cast<double>(__bfloat162float(reinterpret_cast<const __hip_bfloat16*>(buf.data())[idx])) * inv;
-          a.data[(i * a.shape[1] + j) * a.shape[2] + k] = v;
+            for (int64_t k = 0; k < n; ++k)
+              o[k] = static_cast<double>(__bfloat162float(reinterpret_cast<const __hip_bfloat16*>(from)[at + k])) * inv;
+          for (int64_t k = n; k < nk; ++k) o[k] = o[0];
         }
-    });
+      };
+      XF_HIP(out.add(static_cast<const unsigned char*>(fld[c]) + static_cast<size_t>(p0) * plane,
+                     static_cast<size_t>(planes) * plane, planes * nj, static_cast<size_t>(nk) * sizeof(double), put));
+    }
   }
   return XF_OK;
 }
@@ -2114,12 +2124,61 @@ Tiling Engine::tiling() const {
 int Engine::download() {
   if (!uploaded) return fail(XF_ERR_STATE, "download before upload");
   XF_HIP(hipStreamSynchronize(stream));
-  XF_TRY(unpack_fields());
+  {
+    Drain out(stages, stream, plane_bytes(), drain_bytes());
+    XF_HIP(out.open());
+    XF_TRY(drain(out));
+    XF_HIP(out.finish());
+  }
+  return download_rest();
+}
+
+// The fields and the CPML's psi.
+int Engine::drain(Drain& out) {
+  XF_TRY(unpack_fields(out));
   for (size_t q = 0; q < pml_order.size(); ++q) {
     xf_pml& P = sc->pml[pml_order[q]];
     xf_array* ps[4] = {&P.ea_psi_hb, &P.eb_psi_ha, &P.ha_psi_eb, &P.hb_psi_ea};
-    for (int c = 0; c < 4; ++c) XF_TRY(download_c(ps[c]->data, pml[q].psi[c], numel(*ps[c])));
+    for (int c = 0; c < 4; ++c) XF_TRY(drain_c(out, ps[c]->data, pml[q].psi[c], numel(*ps[c])));
   }
+  return XF_OK;
+}
+
+// n values of the compute type
+int Engine::drain_c(Drain& out, double* dst, const void* p, int64_t n) {
+  const bool f64 = plan.precision == XF_FP64;
+  const size_t size = f64 ? sizeof(double) : sizeof(float);
+  const int64_t step = static_cast<int64_t>(out.slot_bytes() / size);
+  constexpr int64_t kRow = 1024;
+  for (int64_t n0 = 0; n0 < n; n0 += step) {
+    const int64_t len = std::min(step, n - n0);
+    double* const to = dst + n0;
+    XF_HIP(out.add(static_cast<const unsigned char*>(p) + static_cast<size_t>(n0) * size, static_cast<size_t>(len) * size,
+                   (len + kRow - 1) / kRow, kRow * sizeof(double),
+                   [=](const unsigned char* from, int64_t lo, int64_t hi) {
+                     const int64_t a = lo * kRow, b = std::min(hi * kRow, len);
+                     if (f64)
+                       std::memcpy(to + a, reinterpret_cast<const double*>(from) + a, static_cast<size_t>(b - a) * sizeof(double));
+                     else
+                       for (int64_t q = a; q < b; ++q) to[q] = reinterpret_cast<const float*>(from)[q];
+                   }));
+  }
+  return XF_OK;
+}
+
+size_t Engine::drain_bytes() const {
+  size_t bytes = 6 * static_cast<size_t>(total) * esize;
+  for (int q : pml_order) {
+    const xf_pml& P = sc->pml[q];
+    for (const xf_array* a : {&P.ea_psi_hb, &P.eb_psi_ha, &P.ha_psi_eb, &P.hb_psi_ea})
+      bytes += static_cast<size_t>(numel(*a)) * (plan.precision == XF_FP64 ? sizeof(double) : sizeof(float));
+  }
+  return bytes;
+}
+
+// What is not drained with the fields and psi: the monitors, the ADE media's
+// and the learned layer's state, and the step.
+int Engine::download_rest() {
   for (int q = 0; q < static_cast<int>(nf.size()); ++q) {
     const xf_nf2ff& N = sc->nf2ff[q];
     const NfPass& P = nf[q].pass;
