@@ -7,13 +7,12 @@
 // scaled inputs x^ = x / s and residual targets r^ = (y - mur) / s, with s
 // and mur exactly as the engine's predictor forms them.
 //
-// Gradient: one thread per sample runs the forward pass with the fp16-
-// rounded weights (fp32 arithmetic) and the backward pass of the mean
-// squared error; every one of the 1505 parameter gradients (and the loss) is
-// summed over the wave's 64 samples with an xor butterfly, accumulated per
-// wave in LDS, summed over the block's waves and written as a per-block
-// partial; a second kernel adds the partials in block order.  Every sum has
-// a fixed order, so a gradient is reproducible bit for bit.
+// Gradient: one lane per sample runs the forward pass with the fp16-rounded
+// weights (fp32 arithmetic) and the backward pass of the mean squared error;
+// the 1505 parameter gradients are summed over a wave's samples on the matrix
+// cores in FP64, over the block's waves in LDS and written as a per-block
+// partial; a second kernel adds the partials.  Every sum has a fixed order,
+// so a gradient is reproducible bit for bit.
 //
 // Optimiser: Adam on fp32 master weights; the forward pass sees them
 // rounded to fp16 (the layer's inference precision), the update is applied
@@ -127,105 +126,160 @@ struct LbRaw {
 // without an index list); the loss is sum d^2 * inv_count.  The weights are
 // the fp16 rounding of w (RoundW: w is fp32 master weights; otherwise w
 // already holds the rounded values).
+//
+// A lane takes a sample through the network in fp32; the parameter gradients
+// are products over the samples, dW2 = gz2^T h1 and dW1 | db1 = gz1^T (x | 1),
+// which the matrix cores form in FP64 from the wave's 64 samples staged in LDS
+// (16x16x4 tiles, products of two fp32 values exact, accumulators in registers
+// over all of a wave's samples); db2, dw3 are column sums of the staged rows,
+// a lane a column.  A butterfly over the wave for each of the 1505 parameters,
+// as before, is some 18000 dependent cross-lane operations a 64 samples:
+// 400 000 samples took 2712 us, now 230 (with k_lb_reduce 2830 and 239).
+// Bound: the forward and backward passes' VALU work, ~5000 instructions a
+// wave and 64 samples.
+typedef double lb_d4 __attribute__((ext_vector_type(4)));
+constexpr int kLbPad = XF_LB_HID + 1;  // floats of a staged row: no two rows of a 4-sample step in the same banks
+
 template <typename Src, bool RoundW>
 __device__ __forceinline__ void lb_grad_body(const Src& src, const uint32_t* __restrict__ idx, int64_t first,
                                              int64_t count, float inv_count, const float* __restrict__ w_in,
                                              float* __restrict__ partial) {
-  __shared__ float w[XF_LB_NPARAM];
-  __shared__ float acc[kLbWaves][kLbAcc];
+  constexpr int H = XF_LB_HID, N = XF_LB_IN;
+  constexpr int ob1 = H * N, oW2 = ob1 + H, ob2 = oW2 + H * H, ow3 = ob2 + H;
+  __shared__ __align__(16) float w[XF_LB_NPARAM];
+  __shared__ __align__(16) float stage[kLbWaves][2][64][kLbPad];
   for (int i = threadIdx.x; i < XF_LB_NPARAM; i += blockDim.x)
     w[i] = RoundW ? __half2float(__float2half_rn(w_in[i])) : w_in[i];
-  for (int i = threadIdx.x; i < kLbWaves * kLbAcc; i += blockDim.x) (&acc[0][0])[i] = 0.0f;
   __syncthreads();
   const float* W1 = w;
-  const float* b1 = W1 + XF_LB_HID * XF_LB_IN;
-  const float* W2 = b1 + XF_LB_HID;
-  const float* b2 = W2 + XF_LB_HID * XF_LB_HID;
-  const float* w3 = b2 + XF_LB_HID;
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  float* a = acc[wave];
+  const float* b1 = W1 + ob1;
+  const float* W2 = w + oW2;
+  const float* b2 = w + ob2;
+  const float* w3 = w + ow3;
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, row = lane / 16, col = lane % 16;
+  float (*const A)[kLbPad] = stage[wave][0];
+  float (*const B)[kLbPad] = stage[wave][1];
+  // what a lane staged, every lane of the wave reads
+  auto staged = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  lb_d4 c2[2][2] = {}, c1[2] = {};
+  double column = 0.0, sum_g = 0.0;  // column: lanes 0..31 db2, 32..63 dw3
+  float sum_l = 0.0f;                 // summed in fp32, the wave's 64 samples as a tree, as ever
   const int64_t stride = (int64_t)gridDim.x * kLbWaves * 64;
   for (int64_t base = ((int64_t)blockIdx.x * kLbWaves + wave) * 64; base < count; base += stride) {
     const int64_t k = base + lane;
     const bool valid = k < count;
-    float x[XF_LB_IN];
+    float x[N];
     float target = 0.0f, lw = 0.0f;
     if (valid) {
       src.get(idx ? (int64_t)idx[k] : first + k, x, target, lw);
     } else {
 #pragma unroll
-      for (int i = 0; i < XF_LB_IN; ++i) x[i] = 0.0f;
+      for (int i = 0; i < N; ++i) x[i] = 0.0f;
     }
-    float h1[XF_LB_HID], h2[XF_LB_HID];
+    float h1[H], h2[H], gz2[H];
 #pragma unroll
-    for (int o = 0; o < XF_LB_HID; ++o) {
+    for (int o = 0; o < H; ++o) {
       float z = b1[o];
 #pragma unroll
-      for (int i = 0; i < XF_LB_IN; ++i) z = z + W1[o * XF_LB_IN + i] * x[i];
+      for (int i = 0; i < N; ++i) z = z + W1[o * N + i] * x[i];
       h1[o] = z > 0.0f ? z : 0.0f;
     }
-    float out = w3[XF_LB_HID];
+    float out = w3[H];
 #pragma unroll
-    for (int o = 0; o < XF_LB_HID; ++o) {
+    for (int o = 0; o < H; ++o) {
       float z = b2[o];
 #pragma unroll
-      for (int i = 0; i < XF_LB_HID; ++i) z = z + W2[o * XF_LB_HID + i] * h1[i];
+      for (int i = 0; i < H; ++i) z = z + W2[o * H + i] * h1[i];
       h2[o] = z > 0.0f ? z : 0.0f;
       out = out + w3[o] * h2[o];
     }
     const float d = out - target;
     const float g_out = valid ? 2.0f * lw * d * inv_count : 0.0f;
-    const float l = valid ? lw * d * d * inv_count : 0.0f;
-    // output layer
-    float s;
-#pragma unroll
-    for (int o = 0; o < XF_LB_HID; ++o) {
-      s = wave_sum(g_out * h2[o]);
-      if (lane == 0) a[XF_LB_HID * XF_LB_IN + XF_LB_HID + XF_LB_HID * XF_LB_HID + XF_LB_HID + o] += s;
-    }
-    s = wave_sum(g_out);
-    if (lane == 0) a[XF_LB_NPARAM - 1] += s;
-    s = wave_sum(l);
-    if (lane == 0) a[XF_LB_NPARAM] += s;
+    sum_g += g_out;
+    sum_l += wave_sum(valid ? lw * d * d * inv_count : 0.0f);
     // second hidden layer
-    float gz2[XF_LB_HID];
 #pragma unroll
-    for (int o = 0; o < XF_LB_HID; ++o) gz2[o] = h2[o] > 0.0f ? g_out * w3[o] : 0.0f;
-    const int oW2 = XF_LB_HID * XF_LB_IN + XF_LB_HID;
-    const int ob2 = oW2 + XF_LB_HID * XF_LB_HID;
-#pragma unroll
-    for (int o = 0; o < XF_LB_HID; ++o) {
-#pragma unroll
-      for (int i = 0; i < XF_LB_HID; ++i) {
-        s = wave_sum(gz2[o] * h1[i]);
-        if (lane == 0) a[oW2 + o * XF_LB_HID + i] += s;
-      }
-      s = wave_sum(gz2[o]);
-      if (lane == 0) a[ob2 + o] += s;
+    for (int o = 0; o < H; ++o) {
+      gz2[o] = h2[o] > 0.0f ? g_out * w3[o] : 0.0f;
+      A[lane][o] = gz2[o];
+      B[lane][o] = h1[o];
     }
-    // first hidden layer
-    const int ob1 = XF_LB_HID * XF_LB_IN;
+    staged();
+#pragma unroll 4
+    for (int q = 0; q < 64; q += 4) {
+      const double a0 = A[q + row][col], a1 = A[q + row][16 + col], e0 = B[q + row][col], e1 = B[q + row][16 + col];
+      c2[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, e0, c2[0][0], 0, 0, 0);
+      c2[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, e1, c2[0][1], 0, 0, 0);
+      c2[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, e0, c2[1][0], 0, 0, 0);
+      c2[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, e1, c2[1][1], 0, 0, 0);
+    }
+    staged();
+    // output layer's products beside gz2: a column sum a lane
 #pragma unroll
-    for (int i = 0; i < XF_LB_HID; ++i) {
+    for (int o = 0; o < H; ++o) B[lane][o] = g_out * h2[o];
+    staged();
+    const float (*const S)[kLbPad] = lane < H ? A : B;
+#pragma unroll 8
+    for (int q = 0; q < 64; ++q) column += (double)S[q][lane % H];
+    staged();
+    // first hidden layer
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
       float g = 0.0f;
 #pragma unroll
-      for (int o = 0; o < XF_LB_HID; ++o) g = g + gz2[o] * W2[o * XF_LB_HID + i];
-      const float gz1 = h1[i] > 0.0f ? g : 0.0f;
-#pragma unroll
-      for (int j = 0; j < XF_LB_IN; ++j) {
-        s = wave_sum(gz1 * x[j]);
-        if (lane == 0) a[i * XF_LB_IN + j] += s;
-      }
-      s = wave_sum(gz1);
-      if (lane == 0) a[ob1 + i] += s;
+      for (int o = 0; o < H; ++o) g = g + gz2[o] * W2[o * H + i];
+      A[lane][i] = h1[i] > 0.0f ? g : 0.0f;
     }
+#pragma unroll
+    for (int j = 0; j < 16; ++j) B[lane][j] = j < N ? x[j < N ? j : 0] : j == N ? 1.0f : 0.0f;
+    staged();
+#pragma unroll 4
+    for (int q = 0; q < 64; q += 4) {
+      const double a0 = A[q + row][col], a1 = A[q + row][16 + col], e = B[q + row][col];
+      c1[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, e, c1[0], 0, 0, 0);
+      c1[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, e, c1[1], 0, 0, 0);
+    }
+    staged();
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) sum_g += __shfl_xor(sum_g, m, 64);
+  // the waves' sums, in the staging rows' place, then the block's
+  __syncthreads();
+  double (*const acc)[kLbAcc] = reinterpret_cast<double (*)[kLbAcc]>(&stage[0][0][0][0]);
+  static_assert(sizeof(double) * kLbWaves * kLbAcc <= sizeof(stage), "the waves' sums fit the staging rows");
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int o = 4 * r + row;  // of a 16x16 FP64 tile a lane holds rows lane / 16 + 4 r of column lane % 16
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) acc[wave][oW2 + (16 * p + o) * H + 16 * q + col] = c2[p][q][r];
+      if (col < N)
+        acc[wave][(16 * p + o) * N + col] = c1[p][r];
+      else if (col == N)
+        acc[wave][ob1 + 16 * p + o] = c1[p][r];
+    }
+  }
+  acc[wave][(lane < H ? ob2 : ow3) + lane % H] = column;
+  if (lane == 0) {
+    acc[wave][XF_LB_NPARAM - 1] = sum_g;
+    acc[wave][XF_LB_NPARAM] = sum_l;
   }
   __syncthreads();
   for (int p = threadIdx.x; p < kLbAcc; p += blockDim.x) {
-    float t = acc[0][p];
+    double t = acc[0][p];
 #pragma unroll
     for (int q = 1; q < kLbWaves; ++q) t += acc[q][p];
-    partial[(int64_t)blockIdx.x * kLbAcc + p] = t;
+    if (p == XF_LB_NPARAM) {
+      float l = (float)acc[0][p];
+#pragma unroll
+      for (int q = 1; q < kLbWaves; ++q) l += (float)acc[q][p];
+      t = l;
+    }
+    partial[(int64_t)blockIdx.x * kLbAcc + p] = (float)t;
   }
 }
 
@@ -272,12 +326,24 @@ __global__ void k_lb_clear_u32(unsigned* __restrict__ p) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *p = 0u;
 }
 
-__global__ void k_lb_reduce(const float* __restrict__ partial, int nblocks, float* __restrict__ grad,
-                            double* __restrict__ loss) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= kLbAcc) return;
+// The blocks' partials, 64 parameters a block: thread row g adds the partials
+// g, g + 16, ... (coalesced over the parameters), the rows are then added in
+// order.  One thread a parameter over all 512 partials was one chain of loads:
+// 121 us.
+constexpr int kLbRows = 16;
+__global__ void __launch_bounds__(64 * kLbRows)
+    k_lb_reduce(const float* __restrict__ partial, int nblocks, float* __restrict__ grad, double* __restrict__ loss) {
+  __shared__ double sum[kLbRows][64];
+  const int lane = threadIdx.x % 64, g = threadIdx.x / 64, p = blockIdx.x * 64 + lane;
   double t = 0.0;
-  for (int b = 0; b < nblocks; ++b) t += (double)partial[(int64_t)b * kLbAcc + p];
+  if (p < kLbAcc)
+#pragma unroll 8
+    for (int b = g; b < nblocks; b += kLbRows) t += (double)partial[(int64_t)b * kLbAcc + p];
+  sum[g][lane] = t;
+  __syncthreads();
+  if (g != 0 || p >= kLbAcc) return;
+#pragma unroll
+  for (int q = 1; q < kLbRows; ++q) t += sum[q][lane];
   if (p < XF_LB_NPARAM)
     grad[p] = (float)t;
   else
@@ -430,7 +496,7 @@ struct LbTrainer {
     const int blocks = static_cast<int>(std::min<int64_t>(nblocks, (count + kLbWaves * 64 - 1) / (kLbWaves * 64)));
     hipLaunchKernelGGL(k_lb_grad, dim3(blocks), dim3(64 * kLbWaves), 0, stream, xs, r, lw, ix, first, count,
                        1.0f / static_cast<float>(count), w16, partial);
-    hipLaunchKernelGGL(k_lb_reduce, dim3((kLbAcc + 255) / 256), dim3(256), 0, stream, partial, blocks, g, loss);
+    hipLaunchKernelGGL(k_lb_reduce, dim3((kLbAcc + 63) / 64), dim3(64 * kLbRows), 0, stream, partial, blocks, g, loss);
     XF_HIP(hipGetLastError());
     return XF_OK;
   }
@@ -541,7 +607,7 @@ int lb_grad_noalloc(const float* raw, int64_t n, double mur_k, int power, const 
   hipLaunchKernelGGL(k_lb_grad_raw, dim3(blocks), dim3(64 * kLbWaves), 0, stream, raw,
                      static_cast<float>(mur_k), power, static_cast<const unsigned*>(absmax), first, count,
                      1.0f / static_cast<float>(count), w32, partial);
-  hipLaunchKernelGGL(k_lb_reduce, dim3((kLbAcc + 255) / 256), dim3(256), 0, stream,
+  hipLaunchKernelGGL(k_lb_reduce, dim3((kLbAcc + 63) / 64), dim3(64 * kLbRows), 0, stream,
                      static_cast<const float*>(partial), blocks, grad, loss);
   XF_HIP(hipGetLastError());
   return XF_OK;
