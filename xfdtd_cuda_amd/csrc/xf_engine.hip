@@ -185,7 +185,7 @@ struct Engine {
   // One pass wherever the scene has the form (step3_tables, step3_incident,
   // step3_faces): on the grids measured it is the faster one or even, us a
   // step against two passes: 536^3 FP64 3765 / 4730, 148^3 FP64 167 / 204,
-  // 50^3 FP64 the least, 253^3 FP32 420 / 419, FP16 storage 423 / 483.
+  // 253^3 FP32 414 / 419, FP16 storage 419 / 483.
   bool use_step3() const { return step3_ready && step3_auto; }
   void step3_swap() {
     std::swap_ranges(fld, fld + 6, fld2);

@@ -27,7 +27,7 @@
 // 4.73 ms).  A block that CPML or a TF/SF face crosses is bound by its waves'
 // chains of dependent scalar, LDS and psi accesses instead, two blocks a CU
 // to hide them (123 to 128 VGPRs in FP64): 148^3 FP64 takes 167 us a step
-// (two passes: 204), 253^3 FP32 420 (419).  Tiles of 6 to 14 rows and 9 to
+// (two passes: 204), 253^3 FP32 414 (419).  Tiles of 6 to 14 rows and 9 to
 // 54 planes a chunk measured within 3 % of each other; loads two planes ahead
 // gained FP64 nothing and cost FP32 its third block a CU (443 -> 497 us on
 // 320^3 without CPML); other block orders (contiguous ranges per XCD, the
