@@ -206,6 +206,7 @@ struct Engine {
   }
   int step3_tables(const std::vector<uint32_t>& ide, const std::vector<uint32_t>& idh);
   bool step3_incident() const;
+  template <typename C>
   bool step3_faces() const;
   int step3_alloc();
   template <typename S>
@@ -1384,7 +1385,8 @@ bool Engine::step3_incident() const {
 // takes at most a quarter of the device memory that is free (the rest is left
 // to other engines and to the caller); without it the two-pass kernels run.
 int Engine::step3_alloc() {
-  if (step3_rows == 0 || !step3_incident() || !step3_faces()) return XF_OK;
+  if (step3_rows == 0 || !step3_incident()) return XF_OK;
+  if (!(plan.precision == XF_FP64 ? step3_faces<double>() : step3_faces<float>())) return XF_OK;
   const size_t kept = allocs.size();
   bool fits = true;
   auto second = [&](void** p, size_t bytes) {
@@ -2876,21 +2878,22 @@ Step3Pass<S> Engine::step3_pass() const {
 
 // Whether k_step3 holds the CPML as it is: faces across one axis so far apart
 // that no node meets two, no plane and its successor two x faces and no block
-// two y faces; and psi arrays that 32-bit byte offsets reach, in rows that 24
-// bits count.
+// two y faces; and psi that the kernel's offsets reach.
+template <typename C>
 bool Engine::step3_faces() const {
   const int gap[3] = {1, kStep3Rows + 2, 0};
   for (int pass = 0; pass < 2; ++pass) {
-    PmlPass<double> P{};
-    fill_pml_pass<double>(*this, P, pass == 1);
+    PmlPass<C> P{};
+    fill_pml_pass<C>(*this, P, pass == 1);
     for (int q = 0; q < P.n; ++q) {
-      const PmlFace<double>& F = P.f[q];
+      const PmlFace<C>& F = P.f[q];
       for (int n = 0; n < q; ++n)
         if (P.f[n].axis == F.axis && P.f[n].c0 < F.c1 + gap[F.axis] && F.c0 < P.f[n].c1 + gap[F.axis]) return false;
+      // the descriptor's fields are 32-bit: the arrays' own sizes first
       const xf_pml& S = sc->pml[pml_order[static_cast<size_t>(q)]];
       for (const xf_array* psi : {&S.ea_psi_hb, &S.eb_psi_ha, &S.ha_psi_eb, &S.hb_psi_ea})
         if (numel(*psi) >= (int64_t(1) << 28)) return false;
-      if (std::max(F.sa2, F.sb2) >= (1 << 24) || ny >= (1 << 24)) return false;
+      if (!step3_face_fits(step3_face<C>(F, pass == 1, F.psi_a, F.psi_b))) return false;
     }
   }
   return true;

@@ -557,7 +557,7 @@ constexpr int kStep3Inc = 192;      // incident values of one table row a block 
 constexpr int kStep3ZJobs = 4;      // TF/SF jobs of z faces a block works out before it marches, a pass
 
 // What a plane's correction by a CPML face of one pass takes, in one scalar
-// load.  psi of node (i, j, k) is at i * plane + j * row + k past the biased
+// load.  psi of node (i, j, k) is step3_psi_offset bytes past the biased
 // pointer (pml_face's layouts for all three axes); psi_a corrects the planes
 // [lo, hi_a), psi_b [lo, hi_b).
 typedef int step3_i16 __attribute__((vector_size(64)));
@@ -591,13 +591,30 @@ struct alignas(64) Step3Job {
   C coef, tr;
 };
 
+// Where psi of node (i, j, k) lies, in bytes from the pointer of a face whose
+// planes begin at lo.  In 32 bits (step3_face_fits), so the planes count from
+// lo: i planes of a far x face are the grid's size, 2^32 bytes from 813^3 in
+// FP64 on.
+template <typename C>
+__host__ __device__ __forceinline__ uint32_t step3_psi_offset(int i, int j, int k, int lo, int row, uint32_t plane) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const uint32_t rows = __umul24(j, row);
+#else
+  const uint32_t rows = ((uint32_t)j & 0xffffffu) * ((uint32_t)row & 0xffffffu);
+#endif
+  return (rows + (uint32_t)k) * (uint32_t)sizeof(C) + (uint32_t)(i - lo) * plane;
+}
+
 // step3_face, step3_job: from the two-pass kernels' descriptors.
 template <typename C>
 Step3Face<C> step3_face(const PmlFace<C>& F, bool is_e, C* oa, C* ob) {
   Step3Face<C> D{};
   const int64_t sa = F.sa1 * F.sa2, sb = F.sb1 * F.sb2;
-  const int64_t ka = F.nstart * (F.axis == 0 ? sa : F.axis == 1 ? F.sa2 : 1);
-  const int64_t kb = F.nstart * (F.axis == 0 ? sb : F.axis == 1 ? F.sb2 : 1);
+  // planes: the main range of an x face; else the lateral range that holds i,
+  // which one of the two psi takes closed and the other half-open
+  D.lo = F.axis == 0 ? F.c0 : F.axis == 1 ? F.b0 : F.a0;
+  const int64_t ka = F.nstart * (F.axis == 0 ? sa : F.axis == 1 ? F.sa2 : 1) - D.lo * sa;
+  const int64_t kb = F.nstart * (F.axis == 0 ? sb : F.axis == 1 ? F.sb2 : 1) - D.lo * sb;
   D.a = F.psi_a - ka;
   D.b = F.psi_b - kb;
   D.oa = oa - ka;
@@ -619,14 +636,25 @@ Step3Face<C> step3_face(const PmlFace<C>& F, bool is_e, C* oa, C* ob) {
   D.off = F.off_c - F.gstart;
   D.ca = F.ca;
   D.cb = F.cb;
-  // planes: the main range of an x face; else the lateral range that holds i,
-  // which one of the two psi takes closed and the other half-open
-  D.lo = F.axis == 0 ? F.c0 : F.axis == 1 ? F.b0 : F.a0;
   const int hi = F.axis == 0 ? F.c1 : F.axis == 1 ? F.b1 : F.a1;
   const bool a_closed = (F.axis == 1) == is_e;
   D.hi_a = F.axis == 0 ? hi : a_closed ? hi + 1 : hi;
   D.hi_b = F.axis == 0 ? hi : a_closed ? hi : hi + 1;
   return D;
+}
+// Whether 32 bits (24 for a row's length and number) hold the offset of every
+// node that the face corrects.
+template <typename C>
+bool step3_face_fits(const Step3Face<C>& D) {
+  const int64_t j = D.axis == 0 ? D.a1 : D.axis == 1 ? D.c1 - 1 : D.b1;
+  const int64_t k = D.axis == 0 ? D.b1 : D.axis == 1 ? D.a1 : D.c1 - 1;
+  const int64_t i = (D.hi_a > D.hi_b ? D.hi_a : D.hi_b) - 1 - D.lo;
+  for (int q = 0; q < 2; ++q) {
+    const int64_t row = q ? D.row_b : D.row_a, plane = q ? D.plane_b : D.plane_a;
+    if (row >= (1 << 24) || j >= (1 << 24)) return false;
+    if ((j * row + k) * static_cast<int64_t>(sizeof(C)) + i * plane >= (int64_t(1) << 32)) return false;
+  }
+  return true;
 }
 template <typename C>
 Step3Job<C> step3_job(const TfsfJob<C>& J, const TfsfPass<C>& T) {

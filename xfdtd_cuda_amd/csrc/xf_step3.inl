@@ -453,8 +453,8 @@ __global__ void __launch_bounds__(64 * (kStep3Rows + 2), 4)
     asm volatile("" : "+s"(u));  // one load, one wait
     const int lo = u[12], hi_a = u[13], hi_b = u[14];
     const unsigned f = bits >> (2 * kMaxPml * ISE + 2 * q);
-    const uint32_t oa = (__umul24(j, u[10]) + (uint32_t)k) * (uint32_t)sizeof(C) + (uint32_t)i * (uint32_t)u[8];
-    const uint32_t ob = (__umul24(j, u[11]) + (uint32_t)k) * (uint32_t)sizeof(C) + (uint32_t)i * (uint32_t)u[9];
+    const uint32_t oa = step3_psi_offset<C>(i, j, k, lo, u[10], (uint32_t)u[8]);
+    const uint32_t ob = step3_psi_offset<C>(i, j, k, lo, u[11], (uint32_t)u[9]);
     auto val = [&](int n, uint32_t o) __attribute__((always_inline)) {
       return gp(reinterpret_cast<C*>(((uint64_t)(uint32_t)u[n] | (uint64_t)(uint32_t)u[n + 1] << 32) + o));
     };
