@@ -68,7 +68,10 @@ struct Batch {
   int step3_blocks{0};
   size_t step3_lds{0};
   bool step3_pml{false};
-  bool step3_fits{false};
+  bool step3_held{false};  // every grid has its second set
+  bool step3_fits{false};  // ... and the launch is described
+  bool take_sets();
+  void drop_sets();
   bool use_step3() const { return step3_auto && step3_fits; }
   int set() const { return inst.empty() ? 0 : inst[0]->eng.step3_set; }
   void swap_sets() {
@@ -102,7 +105,7 @@ struct Batch {
     tf_start[0] = tf_start[1] = nf_start = lb_bstart = lb_mstart = lb_estart = nullptr;
     step3_desc = nullptr;
     step3_start = nullptr;
-    step3_fits = false;
+    step3_held = step3_fits = false;
     pz_items[0] = pz_items[1] = nullptr;
     pz_start[0] = pz_start[1] = nullptr;
     t_dev = nullptr;
@@ -169,6 +172,7 @@ int Batch::create(xf_scene* const* scenes, int n, const xf_plan* pl) {
     if (st != XF_OK) return fail(st, "scene " + std::to_string(g) + ": " + g_err);
     inst.emplace_back(h);
     Engine& E = h->eng;
+    E.in_batch = true;
     if (E.dim != 3) return fail(XF_ERR_UNSUPPORTED, "scene " + std::to_string(g) + ": batches take 3-D grids only");
     if (E.has_ade) return fail(XF_ERR_UNSUPPORTED, "scene " + std::to_string(g) + ": ADE media are not batched");
     // point sources, the learned layer, movies and NF2FF time-domain boxes
@@ -208,6 +212,30 @@ int Batch::upload() {
   return XF_OK;
 }
 
+// Every grid's second set or none, once all of the grids' own arrays are on
+// the device; as Engine::step3_settle, together at most a quarter of what is
+// free then.
+bool Batch::take_sets() {
+  if (step3_held) return true;
+  size_t want = 0, free_bytes = 0, all_bytes = 0;
+  for (auto& h : inst) {
+    if (!h->eng.step3_form) return false;
+    want += h->eng.step3_bytes();
+  }
+  if (hipMemGetInfo(&free_bytes, &all_bytes) != hipSuccess || want > free_bytes / 4) return false;
+  step3_held = true;
+  for (auto& h : inst) step3_held = step3_held && h->eng.step3_take();
+  if (!step3_held) drop_sets();
+  return step3_held;
+}
+
+// The grids' descriptors are to be made again (configure) after it.
+void Batch::drop_sets() {
+  drop_graph();
+  for (auto& h : inst) h->eng.step3_drop();
+  step3_held = step3_fits = false;
+}
+
 namespace {
 template <typename S, typename I, int PM, bool NT>
 int batch_occupancy(int threads) {
@@ -235,6 +263,14 @@ int batch_occupancy_any(int id_bytes, int level, bool nt, int threads) {
                        : batch_occupancy_lv<S, uint16_t>(level, nt, threads);
 }
 }  // namespace
+
+// Items of the two sets, one half after the other; without a second set the
+// same twice, so that the device array holds both whenever a set is taken.
+template <typename T>
+void both_halves(std::vector<T> (&h)[2]) {
+  const std::vector<T>& other = h[1].empty() ? std::vector<T>(h[0]) : h[1];
+  h[0].insert(h[0].end(), other.begin(), other.end());
+}
 
 template <typename S>
 int Batch::configure_t() {
@@ -325,8 +361,7 @@ int Batch::configure_t() {
   }
   // the one-pass step: descriptors of both directions, the blocks of all
   // grids in turn
-  step3_fits = true;
-  for (int g = 0; g < n; ++g) step3_fits = step3_fits && eng(g).step3_ready;
+  step3_fits = step3_held;
   if (step3_fits) {
     std::vector<Step3Pass<S>> desc(2 * static_cast<size_t>(n));
     std::vector<int> start(n + 1, 0);
@@ -349,9 +384,12 @@ int Batch::configure_t() {
     for (int g = 0; g < n; ++g) {
       start[g] = static_cast<int>(blocks);
       blocks += static_cast<int64_t>(desc[g].nkb) * desc[g].njb * desc[g].nch;
-      if (blocks > INT_MAX / 2) return fail(XF_ERR_UNSUPPORTED, "batch too large for 32-bit block ids");
+      if (blocks > INT_MAX / 2) {  // beyond 32-bit block ids: two passes
+        drop_sets();
+        break;
+      }
     }
-    start[n] = step3_blocks = static_cast<int>(blocks);
+    start[n] = step3_blocks = static_cast<int>(std::min<int64_t>(blocks, INT_MAX));
     XF_TRY(put(&step3_desc, desc.data(), desc.size() * sizeof(Step3Pass<S>)));
     void* q = step3_start;
     XF_TRY(put(&q, start.data(), start.size() * sizeof(int)));
@@ -386,7 +424,7 @@ int Batch::configure_t() {
       }
     }
     });
-    halves[0].insert(halves[0].end(), halves[1].begin(), halves[1].end());
+    both_halves(halves);
     n_nf = static_cast<int>(st.size()) - 1;
     nf_total = st.back();
     XF_TRY(put(&nf_items, items.data(), items.size() * sizeof(NfItem<S>)));
@@ -410,7 +448,7 @@ int Batch::configure_t() {
       ++n_pt;
     }
     });
-    halves[0].insert(halves[0].end(), halves[1].begin(), halves[1].end());
+    both_halves(halves);
     XF_TRY(put(&pt_items, items.data(), items.size() * sizeof(PointItem<S>)));
   }
   {
@@ -437,7 +475,7 @@ int Batch::configure_t() {
       lb_any_record = lb_any_record || !apply;
     }
     });
-    halves[0].insert(halves[0].end(), halves[1].begin(), halves[1].end());
+    both_halves(halves);
     lb_edges = se.back();
     n_lb = static_cast<int>(st.size()) - 1;
     lb_blocks = st.back();
@@ -470,6 +508,7 @@ int Batch::configure() {
   if (tune.blocks < 0) return fail(XF_ERR_INVALID, "blocks must be >= 0");
   XF_HIP(hipSetDevice(device));
   drop_graph();
+  if (step3_auto) (void)take_sets();
   int st;
   switch (plan.precision) {
     case XF_FP64: st = configure_t<double>(); break;
@@ -779,7 +818,7 @@ int Batch::autotune(int trial_steps, xf_tuning* best) {
   const bool keep_auto = step3_auto;
   bool win_step3 = false;
   step3_auto = true;
-  if (step3_fits) {
+  if (take_sets()) {
     tune = xf_tuning{1, 4, 0, 1, 0, 1, 0, 0.0};
     status = configure();
     if (status == XF_OK) status = run(1);
@@ -841,6 +880,7 @@ int Batch::autotune(int trial_steps, xf_tuning* best) {
     return status;
   }
   tune = win;
+  if (!win_step3) drop_sets();
   XF_TRY(configure());
   if (best) *best = win;
   return XF_OK;
@@ -873,8 +913,11 @@ int Engine::autotune(int trial_steps, xf_tuning* best) {
   pml_ztail = keep_tail;
   // the one-pass step, then the two-pass tilings
   bool win_step3 = false;
-  if (step3_ready) {
+  if (step3_form) {
     set_tiling(0, 0, 0);
+    step3_settle();
+  }
+  if (step3_ready) {
     status = run(1);
     if (status == XF_OK) status = run(trial_steps);
     if (status == XF_OK) {
@@ -925,6 +968,7 @@ int Engine::autotune(int trial_steps, xf_tuning* best) {
     set_tiling(0, 0, 0);
     return XF_OK;
   }
+  step3_drop();
   set_tiling(win.tile_y, static_cast<int>((nx + 1 + win.planes - 1) / win.planes),
              XF_TILE_SET | (win.nontemporal ? XF_TILE_NT : 0) | (win.pml_split == 1 ? XF_TILE_PML_SPLIT : 0) |
                  (win.pml_split == 2 ? XF_TILE_PML_ZTAIL : 0) | (win.k32 ? XF_TILE_K32 : 0));
@@ -1009,6 +1053,7 @@ int xf_batch_set_tuning(xf_batch* b, const xf_tuning* t) {
       return xf::fail(XF_ERR_INVALID, "bad tuning (tile_y 1..4, planes >= 1, blocks >= 0, pml_split 0..2)");
     }
     if (!b->b.uploaded) return XF_OK;
+    b->b.drop_sets();
     const int st = b->b.configure();
     if (st != XF_OK) {
       b->b.tune = keep;

@@ -172,11 +172,15 @@ struct Engine {
   // each launch, so fld and psi always name the current ones.  step3_set
   // counts the swaps modulo two: the descriptor a launch takes.
   void* fld2[6]{};
-  bool step3_ready{false};  // the scene has the one-pass form (tables and second set on the device)
+  bool step3_form{false};   // the scene has the one-pass form
+  bool step3_ready{false};  // ... and its tables and the second set are on the device
   bool step3_auto{true};    // the tiling was left to the engine
   int step3_set{0};
-  void* step3_ids{};        // one byte per node: row of step3_tab
-  void* step3_tab{};        // 18 coefficients per pair of E and H rows
+  bool in_batch{false};     // the batch decides on the second set
+  std::vector<uint8_t> step3_ids_h;  // one byte per node: row of step3_tab
+  std::vector<double> step3_tab_h;   // 18 coefficients per pair of E and H rows
+  void* step3_ids{};
+  void* step3_tab{};
   int step3_rows{0};
   uint64_t step3_dmask{0};
   void* step3_desc{};       // two Step3Pass, one per direction
@@ -204,15 +208,20 @@ struct Engine {
         if (p == D.psi[2 + q] || p == D.psi2[q]) return D.psi[2 + q];
     return p;
   }
-  int step3_tables(const std::vector<uint32_t>& ide, const std::vector<uint32_t>& idh);
+  void step3_tables(const std::vector<uint32_t>& ide, const std::vector<uint32_t>& idh);
   bool step3_incident() const;
   template <typename C>
   bool step3_faces() const;
-  int step3_alloc();
+  size_t step3_psi_bytes(size_t q, int c) const;
+  size_t step3_bytes() const;
+  bool step3_take();
+  void step3_drop();
+  void step3_forget();
+  void step3_settle();
   template <typename S>
   Step3Pass<S> step3_pass() const;
   template <typename S>
-  int step3_describe();
+  bool step3_describe();
   size_t step3_lds() const { return static_cast<size_t>(step3_rows) * 18 * (plan.precision == XF_FP64 ? 8 : 4); }
   template <typename S>
   int launch_step3(int t, const int* tp);
@@ -325,6 +334,7 @@ struct Engine {
   bool use_lists() const { return pml_streams && dim == 3 && !dense && tlist[0] && tlist[1]; }
   int rows() const { return tile_y * (64 / klanes); }  // j-rows of a block
   void set_tiling(int ty, int chunks_x, int flags);
+  void describe_layout();
   Tiling tiling() const;
   int snapshot();  // copy every state buffer aside (device to device)
   int restore();   // put the copies back; the step counter is the caller's
@@ -350,8 +360,10 @@ struct Engine {
     state.clear();
     backup.clear();
     std::fill(fld2, fld2 + 6, nullptr);
-    step3_ready = false;
+    step3_form = step3_ready = false;
     step3_set = 0;
+    step3_ids_h = {};
+    step3_tab_h = {};
     step3_ids = step3_tab = step3_desc = nullptr;
     step3_start = nullptr;
     if (stream) (void)hipStreamDestroy(stream);
@@ -1310,16 +1322,17 @@ int Engine::build_ids() {
           if (disp[(i * ny + j) * nz + k]) ade_cells.push_back((i * (ny + 1) + j) * (nz + 1) + k);
   }
   match_cpsi(ide, idh);
-  return step3_tables(ide, idh);
+  step3_tables(ide, idh);
+  return XF_OK;
 }
 
 // The one-pass step's ids: the pairs of E and H rows that occur, (0, 0)
 // first (a node that is no cell has row 0 in both tables).  Its blocks hold
 // the whole table in LDS, so a scene with more than kStep3MaxRows pairs, or
 // dense coefficients, keeps the two-pass kernels.
-int Engine::step3_tables(const std::vector<uint32_t>& ide, const std::vector<uint32_t>& idh) {
+void Engine::step3_tables(const std::vector<uint32_t>& ide, const std::vector<uint32_t>& idh) {
   step3_rows = 0;
-  if (dense || dim != 3 || sy >= (int64_t(1) << 24) || ntab_e > kStep3MaxRows || ntab_h > kStep3MaxRows) return XF_OK;
+  if (dense || dim != 3 || sy >= (int64_t(1) << 24) || ntab_e > kStep3MaxRows || ntab_h > kStep3MaxRows) return;
   const size_t most = has_ade ? kStep3AdeRows : kStep3MaxRows;
   std::vector<int> at(static_cast<size_t>(ntab_e) * ntab_h, -1);
   std::vector<std::pair<int, int>> pairs{{0, 0}};
@@ -1334,7 +1347,7 @@ int Engine::step3_tables(const std::vector<uint32_t>& ide, const std::vector<uin
       lh = idh[c];
       int& p = at[static_cast<size_t>(le) * ntab_h + lh];
       if (p < 0) {
-        if (pairs.size() >= most) return XF_OK;
+        if (pairs.size() >= most) return;
         p = static_cast<int>(pairs.size());
         pairs.emplace_back(static_cast<int>(le), static_cast<int>(lh));
       }
@@ -1342,20 +1355,17 @@ int Engine::step3_tables(const std::vector<uint32_t>& ide, const std::vector<uin
     }
     id[c] = static_cast<uint8_t>(run_end);
   }
-  std::vector<double> tab;
   step3_dmask = 0;
   for (size_t q = 0; q < pairs.size(); ++q) {
-    for (int n = 0; n < 9; ++n) tab.push_back(etab_h[static_cast<size_t>(pairs[q].first) * 9 + n]);
-    for (int n = 0; n < 9; ++n) tab.push_back(htab_h[static_cast<size_t>(pairs[q].second) * 9 + n]);
+    for (int n = 0; n < 9; ++n) step3_tab_h.push_back(etab_h[static_cast<size_t>(pairs[q].first) * 9 + n]);
+    for (int n = 0; n < 9; ++n) step3_tab_h.push_back(htab_h[static_cast<size_t>(pairs[q].second) * 9 + n]);
     if (has_ade && eflag_h[pairs[q].first]) step3_dmask |= uint64_t(1) << q;
   }
-  XF_TRY(upload_c(&step3_tab, tab.data(), static_cast<int64_t>(tab.size())));
   step3_rows = static_cast<int>(pairs.size());
-  std::vector<uint8_t> v(total, 0);
+  step3_ids_h.assign(total, 0);
   for (int64_t i = 0; i < nx; ++i)
     for (int64_t j = 0; j < ny; ++j)
-      std::copy_n(id.data() + (i * ny + j) * nz, nz, v.data() + i * sx + j * sy);
-  return upload_vec(&step3_ids, v);
+      std::copy_n(id.data() + (i * ny + j) * nz, nz, step3_ids_h.data() + i * sx + j * sy);
 }
 
 // Whether a block's share of the incident tables is bounded as k_step3 holds
@@ -1381,57 +1391,111 @@ bool Engine::step3_incident() const {
   return true;
 }
 
-// The second set of fields and H-pass psi, a copy of the first, where it
-// takes at most a quarter of the device memory that is free (the rest is left
-// to other engines and to the caller); without it the two-pass kernels run.
-int Engine::step3_alloc() {
-  if (step3_rows == 0 || !step3_incident()) return XF_OK;
-  if (!(plan.precision == XF_FP64 ? step3_faces<double>() : step3_faces<float>())) return XF_OK;
+size_t Engine::step3_psi_bytes(size_t q, int c) const {
+  const xf_pml& P = sc->pml[pml_order[q]];
+  return static_cast<size_t>(numel(c == 0 ? P.ha_psi_eb : P.hb_psi_ea)) * (plan.precision == XF_FP64 ? 8 : 4);
+}
+
+// What the one-pass step takes of the device beyond the two-pass kernels: the
+// second set of fields and H-pass psi, the ids and the table.
+size_t Engine::step3_bytes() const {
+  size_t n = 6 * static_cast<size_t>(total) * esize + static_cast<size_t>(total) + step3_lds();
+  for (size_t q = 0; q < pml.size(); ++q) n += step3_psi_bytes(q, 0) + step3_psi_bytes(q, 1);
+  return n;
+}
+
+// Takes them, the second set a copy of the first.  False, with nothing taken,
+// if the scene lacks the form or the device the memory.
+bool Engine::step3_take() {
+  if (step3_ready || !step3_form) return step3_ready;
   const size_t kept = allocs.size();
-  bool fits = true;
-  auto second = [&](void** p, size_t bytes) {
+  bool ok = hipSetDevice(device) == hipSuccess;
+  auto take = [&](void** p, size_t bytes) {
     *p = nullptr;
-    if (!fits) return;
-    if (hipMalloc(p, bytes ? bytes : 16) != hipSuccess) {
-      (void)hipGetLastError();
-      *p = nullptr;
-      fits = false;
-      return;
-    }
-    allocs.push_back(*p);
+    if (!ok) return;
+    ok = hipMalloc(p, bytes ? bytes : 16) == hipSuccess;
+    if (!ok) *p = nullptr;
+    if (ok) allocs.push_back(*p);
   };
-  auto psi_bytes = [&](size_t q, int c) {
-    const xf_pml& P = sc->pml[pml_order[q]];
-    return static_cast<size_t>(numel(c == 0 ? P.ha_psi_eb : P.hb_psi_ea)) * (plan.precision == XF_FP64 ? 8 : 4);
+  auto copy = [&](void* to, const void* from, size_t bytes, hipMemcpyKind kind) {
+    ok = ok && hipMemcpyAsync(to, from, bytes, kind, stream) == hipSuccess;
   };
-  size_t want = 6 * static_cast<size_t>(total) * esize, free_bytes = 0, all_bytes = 0;
-  for (size_t q = 0; q < pml.size(); ++q) want += psi_bytes(q, 0) + psi_bytes(q, 1);
-  XF_HIP(hipMemGetInfo(&free_bytes, &all_bytes));
-  if (want > free_bytes / 4) return XF_OK;
-  for (int c = 0; c < 6; ++c) second(&fld2[c], static_cast<size_t>(total) * esize);
+  for (int c = 0; c < 6; ++c) take(&fld2[c], static_cast<size_t>(total) * esize);
   for (size_t q = 0; q < pml.size(); ++q)
-    for (int c = 0; c < 2; ++c) second(&pml[q].psi2[c], psi_bytes(q, c));
-  if (!fits) {
+    for (int c = 0; c < 2; ++c) take(&pml[q].psi2[c], step3_psi_bytes(q, c));
+  take(&step3_ids, step3_ids_h.size());
+  take(&step3_tab, step3_lds());
+  for (int c = 0; c < 6; ++c) copy(fld2[c], fld[c], static_cast<size_t>(total) * esize, hipMemcpyDeviceToDevice);
+  for (size_t q = 0; q < pml.size(); ++q)
+    for (int c = 0; c < 2; ++c) copy(pml[q].psi2[c], pml[q].psi[2 + c], step3_psi_bytes(q, c), hipMemcpyDeviceToDevice);
+  copy(step3_ids, step3_ids_h.data(), step3_ids_h.size(), hipMemcpyHostToDevice);
+  const std::vector<float> tab32(step3_tab_h.begin(), step3_tab_h.end());
+  copy(step3_tab, plan.precision == XF_FP64 ? static_cast<const void*>(step3_tab_h.data()) : tab32.data(), step3_lds(),
+       hipMemcpyHostToDevice);
+  ok = ok && hipStreamSynchronize(stream) == hipSuccess;
+  step3_set = 0;
+  if (ok && !in_batch) {  // a batch has descriptors of its own
+    void* start = nullptr;
+    take(&step3_desc, 2 * sizeof(Step3Pass<double>));
+    take(&start, 2 * sizeof(int));
+    step3_start = static_cast<int*>(start);
+    if (ok) switch (plan.precision) {
+        case XF_FP64: ok = step3_describe<double>(); break;
+        case XF_FP32: ok = step3_describe<float>(); break;
+        case XF_BF16_COMP: ok = step3_describe<Bf16c>(); break;
+        case XF_FP16_STORE: ok = step3_describe<__half>(); break;
+        default: ok = step3_describe<__hip_bfloat16>();
+      }
+  }
+  step3_ready = ok;
+  if (!ok) {
+    (void)hipGetLastError();
     for (size_t q = kept; q < allocs.size(); ++q) (void)hipFree(allocs[q]);
     allocs.resize(kept);
-    std::fill(fld2, fld2 + 6, nullptr);
-    for (PmlDev& D : pml) D.psi2[0] = D.psi2[1] = nullptr;
-    return XF_OK;
+    step3_forget();
   }
-  for (int c = 0; c < 6; ++c)
-    XF_HIP(hipMemcpyAsync(fld2[c], fld[c], static_cast<size_t>(total) * esize, hipMemcpyDeviceToDevice, stream));
-  for (size_t q = 0; q < pml.size(); ++q)
-    for (int c = 0; c < 2; ++c)
-      XF_HIP(hipMemcpyAsync(pml[q].psi2[c], pml[q].psi[2 + c], psi_bytes(q, c), hipMemcpyDeviceToDevice, stream));
-  XF_HIP(hipStreamSynchronize(stream));
-  step3_ready = true;
-  switch (plan.precision) {
-    case XF_FP64: return step3_describe<double>();
-    case XF_FP32: return step3_describe<float>();
-    case XF_BF16_COMP: return step3_describe<Bf16c>();
-    case XF_FP16_STORE: return step3_describe<__half>();
-    default: return step3_describe<__hip_bfloat16>();
+  return ok;
+}
+
+void Engine::step3_forget() {
+  std::fill(fld2, fld2 + 6, nullptr);
+  for (PmlDev& D : pml) D.psi2[0] = D.psi2[1] = nullptr;
+  step3_ids = step3_tab = step3_desc = nullptr;
+  step3_start = nullptr;
+  step3_set = 0;
+  step3_ready = false;
+}
+
+// Gives them back.  The set the fields are in now stays, whichever it is.
+void Engine::step3_drop() {
+  if (!step3_ready) return;
+  drop_graph();
+  for (auto& s : state) s.first = live(s.first);
+  std::vector<void*> gone(fld2, fld2 + 6);
+  for (PmlDev& D : pml) gone.insert(gone.end(), D.psi2, D.psi2 + 2);
+  for (void* p : {step3_ids, step3_tab, step3_desc, static_cast<void*>(step3_start)})
+    if (p) gone.push_back(p);
+  for (void* p : gone) {
+    (void)hipFree(p);
+    allocs.erase(std::find(allocs.begin(), allocs.end(), p));
   }
+  step3_forget();
+}
+
+// The second set is held where the step uses it: the tiling was left to the
+// engine and the set takes at most a quarter of the device memory that is
+// free (the rest is left to other engines and to the caller).
+void Engine::step3_settle() {
+  if (in_batch || !stream) return;
+  if (!step3_auto) {
+    step3_drop();
+  } else if (step3_form && !step3_ready) {
+    size_t free_bytes = 0, all_bytes = 0;
+    if (hipSetDevice(device) == hipSuccess && hipMemGetInfo(&free_bytes, &all_bytes) == hipSuccess &&
+        step3_bytes() <= free_bytes / 4)
+      (void)step3_take();
+  }
+  describe_layout();
 }
 
 // The c_psi value of a corrected node is the curl coefficient, along the
@@ -2012,8 +2076,10 @@ int Engine::upload() {
   t_dev = static_cast<int*>(tp);
   XF_TRY(alloc(&tp, 64));
   wd_dev = static_cast<unsigned*>(tp);
-  XF_TRY(step3_alloc());
+  step3_form = step3_rows > 0 && step3_incident() &&
+               (plan.precision == XF_FP64 ? step3_faces<double>() : step3_faces<float>());
   set_tiling(plan.tile_y, plan.chunks_x, plan.tiling_flags);
+  step3_settle();
   XF_HIP(hipDeviceSynchronize());
   uploaded = true;
   return XF_OK;
@@ -2072,6 +2138,10 @@ void Engine::set_tiling(int ty, int chunks_x, int flags) {
   }
   drop_graph();
   if (pml_streams && dim == 3 && stream && build_tile_lists() != XF_OK) pml_streams = 0;
+  describe_layout();
+}
+
+void Engine::describe_layout() {
   layout_desc = std::string("dim=") + std::to_string(dim) + " pad_stride=" + std::to_string(dim == 3 ? sy : sx) +
                 " id_bytes=" + std::to_string(id_bytes) + " coeff=" + (dense ? "dense" : "table") +
                 " etab=" + std::to_string(ntab_e) +
@@ -2926,7 +2996,7 @@ int step3_pick_chunk(const std::vector<const Engine*>& grids, bool pml, size_t l
 }
 
 template <typename S>
-int Engine::step3_describe() {
+bool Engine::step3_describe() {
   step3_chunk = step3_pick_chunk<S>({this}, !pml.empty(), step3_lds());
   Step3Pass<S> D[2];
   D[0] = step3_pass<S>();
@@ -2934,19 +3004,12 @@ int Engine::step3_describe() {
   D[1] = step3_pass<S>();
   step3_swap();
   const int64_t blocks = static_cast<int64_t>(D[0].nkb) * D[0].njb * D[0].nch;
-  if (blocks > INT_MAX / 2) {
-    step3_ready = false;
-    return XF_OK;
-  }
+  if (blocks > INT_MAX / 2) return false;
   step3_blocks = static_cast<int>(blocks);
-  XF_TRY(alloc(&step3_desc, sizeof(D)));
-  XF_HIP(hipMemcpy(step3_desc, D, sizeof(D), hipMemcpyHostToDevice));
   const int start[2] = {0, step3_blocks};
-  void* p = nullptr;
-  XF_TRY(alloc(&p, sizeof(start)));
-  step3_start = static_cast<int*>(p);
-  XF_HIP(hipMemcpy(step3_start, start, sizeof(start), hipMemcpyHostToDevice));
-  return XF_OK;
+  static_assert(sizeof(Step3Pass<S>) <= sizeof(Step3Pass<double>), "step3_take's allocation");
+  return hipMemcpy(step3_desc, D, sizeof(D), hipMemcpyHostToDevice) == hipSuccess &&
+         hipMemcpy(step3_start, start, sizeof(start), hipMemcpyHostToDevice) == hipSuccess;
 }
 
 // One step from the current set into the other, which becomes current.
@@ -3374,6 +3437,7 @@ int xf_set_tiling(xf_handle* h, int32_t tile_y, int32_t chunks_x, int32_t flags)
     // the Yee kernels are compiled for at most 256 threads per block (64 x 4)
     if (tile_y < 0 || tile_y > 4 || chunks_x < 0) return xf::fail(XF_ERR_INVALID, "bad tiling (tile_y 0..4)");
     h->eng.set_tiling(tile_y, chunks_x, flags);
+    h->eng.step3_settle();
     return XF_OK;
   });
 }
