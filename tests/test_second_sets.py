@@ -146,3 +146,94 @@ def test_no_second_set_in_a_batch_with_a_grid_that_lacks_the_form(fake):
     assert step3(b) and fake.fake_used() == held
     b.close()
     """)
+
+
+def test_a_failing_allocation_has_idle_handles_give_theirs_back(fake):
+    """Handles that fit the device without second sets all fit it, whichever
+    came first, and go on stepping."""
+    _run(fake, """
+    bare = cost(lambda: xf.Engine(scene(24), tile_y=1).upload())
+    fake.fake_limit(int(8.2 * bare))
+    sims = [scene(24, q) for q in range(9)]
+    want = [saved(s) for s in sims]
+    e = [xf.Engine(sims[0], use_graph=True).upload(), xf.Engine(sims[1]).upload()]
+    assert step3(e[0]) and step3(e[1])
+    e[0].run(3)  # its fields are in the second set, which stays
+    e[1].run(2)
+    b = xf.Batch(sims[2:4]).upload()
+    assert step3(b) == (2 * bare < (8.2 - 5.5) / 4 * bare)
+    for s in sims[4:8]:
+        e.append(xf.Engine(s).upload())
+    assert not step3(e[0]) and not step3(e[1]) and not step3(e[-1])
+    try:
+        xf.Engine(sims[8]).upload()
+        raise SystemExit("nine grids cannot fit")
+    except xf.XFError as err:
+        assert "status 5" in str(err), err
+    for x in e + [b]:
+        x.run(3).run(2).download()
+    for s, w in zip(sims[:8], want):
+        assert all(np.array_equal(x, y) for x, y in zip(saved(s), w))
+    e.pop().close()
+    e[0].set_tiling()  # room again
+    fake.fake_limit(1 << 40)
+    e[0].set_tiling()
+    assert step3(e[0])
+    """)
+
+
+def test_a_batch_gives_its_sets_back(fake):
+    _run(fake, """
+    bare = cost(lambda: xf.Batch([scene(24, q) for q in range(3)]).set_tuning(tile_y=1).upload())
+    sims = [scene(24, q) for q in range(6)]
+    want = [saved(s) for s in sims]
+    fake.fake_limit(5 * bare)
+    b = xf.Batch(sims[:3], use_graph=True).upload()
+    assert step3(b)
+    b.run(3)
+    fake.fake_limit(int(2.1 * bare))
+    c = xf.Batch(sims[3:]).upload()
+    assert not step3(b) and not step3(c)
+    b.run(2).run(3).download()
+    c.run(2).download()
+    for s, w in zip(sims, want):
+        assert all(np.array_equal(x, y) for x, y in zip(saved(s), w))
+    c.close()
+    # its own snapshots come before its second sets
+    fake.fake_limit(5 * bare)
+    b.upload()
+    assert step3(b)
+    fake.fake_limit(int(2.1 * bare))
+    b.autotune(2)
+    assert not step3(b)
+    b.run(3).download()
+    for s, w in zip(sims[:3], want):
+        assert all(np.array_equal(x, y) for x, y in zip(saved(s), w))
+    """)
+
+
+def test_threads_fill_the_device(fake):
+    """Handles made, run and closed by several threads under a limit that is
+    short of second sets for all."""
+    _run(fake, """
+    import threading
+    bare = cost(lambda: xf.Engine(scene(16), tile_y=1).upload())
+    fake.fake_limit(int(5.5 * bare))
+    errors = []
+    def work(q):
+        try:
+            for turn in range(12):
+                s = scene(16, q)
+                w = saved(s)
+                e = xf.Engine(s).upload()
+                e.run(3).describe()
+                e.run(2).download()
+                assert all(np.array_equal(x, y) for x, y in zip(saved(s), w))
+                e.close()
+        except Exception as err:
+            errors.append(repr(err))
+    ts = [threading.Thread(target=work, args=(q,)) for q in range(4)]
+    for t in ts: t.start()
+    for t in ts: t.join()
+    assert not errors, errors
+    """)

@@ -16,7 +16,7 @@
 
 namespace xf {
 
-struct Batch {
+struct Batch : SecondSet {
   std::vector<std::unique_ptr<xf_handle>> inst;
   xf_plan plan{};
   int device{0};
@@ -68,10 +68,13 @@ struct Batch {
   int step3_blocks{0};
   size_t step3_lds{0};
   bool step3_pml{false};
-  bool step3_held{false};  // every grid has its second set
-  bool step3_fits{false};  // ... and the launch is described
+  std::atomic<bool> step3_held{false};  // every grid has its second set
+  std::atomic<bool> step3_fits{false};  // ... and the launch is described
+  bool stale{false};  // the sets were given back: the descriptors are to be made again
   bool take_sets();
   void drop_sets();
+  void give_back() override;
+  void describe();
   bool use_step3() const { return step3_auto && step3_fits; }
   int set() const { return inst.empty() ? 0 : inst[0]->eng.step3_set; }
   void swap_sets() {
@@ -82,6 +85,7 @@ struct Batch {
   bool graph_ready{false};
   xf_timing timing{};
   std::string desc;
+  mutable std::mutex desc_m;
 
   ~Batch() { release(); }
 
@@ -96,6 +100,7 @@ struct Batch {
   }
 
   void release() {
+    SecondSets::all().remove(this);
     drop_graph();
     for (void* p : allocs) (void)hipFree(p);
     allocs.clear();
@@ -116,7 +121,7 @@ struct Batch {
 
   int alloc(void** p, size_t bytes) {
     *p = nullptr;
-    hipError_t e = hipMalloc(p, bytes ? bytes : 16);
+    hipError_t e = SecondSets::all().malloc(p, bytes ? bytes : 16, device, this);
     if (e != hipSuccess) return fail(XF_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     allocs.push_back(*p);
     return XF_OK;
@@ -172,7 +177,7 @@ int Batch::create(xf_scene* const* scenes, int n, const xf_plan* pl) {
     if (st != XF_OK) return fail(st, "scene " + std::to_string(g) + ": " + g_err);
     inst.emplace_back(h);
     Engine& E = h->eng;
-    E.in_batch = true;
+    E.batch = this;
     if (E.dim != 3) return fail(XF_ERR_UNSUPPORTED, "scene " + std::to_string(g) + ": batches take 3-D grids only");
     if (E.has_ade) return fail(XF_ERR_UNSUPPORTED, "scene " + std::to_string(g) + ": ADE media are not batched");
     // point sources, the learned layer, movies and NF2FF time-domain boxes
@@ -223,17 +228,28 @@ bool Batch::take_sets() {
     want += h->eng.step3_bytes();
   }
   if (hipMemGetInfo(&free_bytes, &all_bytes) != hipSuccess || want > free_bytes / 4) return false;
-  step3_held = true;
-  for (auto& h : inst) step3_held = step3_held && h->eng.step3_take();
-  if (!step3_held) drop_sets();
-  return step3_held;
+  bool all = true;
+  for (auto& h : inst) all = all && h->eng.step3_take();
+  step3_held = all;
+  if (all)
+    SecondSets::all().add(this, device, want);
+  else
+    for (auto& h : inst) h->eng.step3_drop();
+  return all;
 }
 
 // The grids' descriptors are to be made again (configure) after it.
 void Batch::drop_sets() {
+  SecondSets::all().remove(this);
+  give_back();
+}
+
+void Batch::give_back() {
   drop_graph();
   for (auto& h : inst) h->eng.step3_drop();
   step3_held = step3_fits = false;
+  stale = true;
+  describe();
 }
 
 namespace {
@@ -361,7 +377,7 @@ int Batch::configure_t() {
   }
   // the one-pass step: descriptors of both directions, the blocks of all
   // grids in turn
-  step3_fits = step3_held;
+  step3_fits = step3_held.load();
   if (step3_fits) {
     std::vector<Step3Pass<S>> desc(2 * static_cast<size_t>(n));
     std::vector<int> start(n + 1, 0);
@@ -518,11 +534,17 @@ int Batch::configure() {
     default: st = configure_t<__hip_bfloat16>(); break;
   }
   if (st != XF_OK) return st;
+  stale = false;
+  describe();
+  return XF_OK;
+}
+
+void Batch::describe() {
   // grids whose every c_psi value the tiles read from the coefficient table
   int cpsi_tab = 0;
   for (size_t g = 0; g < inst.size(); ++g)
     cpsi_tab += eng(static_cast<int>(g)).cpsi_matched() == 4 * static_cast<int>(eng(static_cast<int>(g)).pml.size()) ? 1 : 0;
-  desc = "grids=" + std::to_string(inst.size()) + " cells=" + std::to_string(cells) +
+  const std::string d = "grids=" + std::to_string(inst.size()) + " cells=" + std::to_string(cells) +
          " tiles=" + std::to_string(total_tiles) + " blocks=" + std::to_string(grid_blocks) +
          " resident=" + std::to_string(resident) + " tile_y=" + std::to_string(tune.tile_y) +
          " planes=" + std::to_string(tune.planes) + " nt=" + std::to_string(tune.nontemporal) +
@@ -532,7 +554,8 @@ int Batch::configure() {
          " tfsf=" + std::to_string(n_tf[0]) +
          " nf2ff=" + std::to_string(n_nf) + " cpsi_tab=" + std::to_string(cpsi_tab) +
          " step3=" + std::to_string(use_step3() ? 1 : 0) + (use_step3() ? " step3_blocks=" + std::to_string(step3_blocks) : std::string());
-  return XF_OK;
+  std::lock_guard<std::mutex> lock(desc_m);
+  desc = d;
 }
 
 template <typename S>
@@ -635,6 +658,7 @@ int Batch::run(int64_t n) {
   if (nt != INT64_MAX && cur_step + n > nt)
     return fail(XF_ERR_INVALID, "run past the end of the time axis the TFSF/NF2FF tables were built for");
   XF_HIP(hipSetDevice(device));
+  if (stale) XF_TRY(configure());
   const bool timing_on = plan.timing != 0;
   const bool graph_on = plan.use_graph != 0 && !timing_on;
   auto step = [&](int t, bool tdev, bool ev_on, hipEvent_t* e) -> int {
@@ -776,7 +800,12 @@ int Batch::download() {
 }
 
 int Batch::snapshot() {
-  for (auto& h : inst) XF_TRY(h->eng.snapshot());
+  for (auto& h : inst) {
+    const int st = h->eng.snapshot();
+    if (st == XF_OK) continue;
+    for (auto& done : inst) done->eng.drop_backup();
+    return st;
+  }
   return XF_OK;
 }
 
@@ -794,14 +823,18 @@ int Batch::autotune(int trial_steps, xf_tuning* best) {
   if (trial_steps < 1) return fail(XF_ERR_INVALID, "trial_steps must be >= 1");
   if (nt != INT64_MAX && cur_step + trial_steps + 1 > nt)
     return fail(XF_ERR_INVALID, "not enough time-table steps left to tune");
-  XF_TRY(snapshot());
+  int status = snapshot();
+  if (status == XF_ERR_NOMEM && step3_held) {  // no room for both
+    drop_sets();
+    status = snapshot();
+  }
+  if (status != XF_OK) return status;
   const int64_t step0 = cur_step;
   const xf_timing keep = timing;
   const int keep_timing = plan.timing;
   plan.timing = 0;
   xf_tuning win{};
   win.step_ms = 1e30;
-  int status = XF_OK;
   // the z-face split and tail only where some grid can take them
   bool can_split = false, can_tail = false;
   for (auto& h : inst) {
@@ -892,14 +925,19 @@ int Engine::autotune(int trial_steps, xf_tuning* best) {
   if (trial_steps < 1) return fail(XF_ERR_INVALID, "trial_steps must be >= 1");
   if ((sc->tfsf || !nf.empty() || !nftd.empty() || pts.n > 0) && cur_step + trial_steps + 1 > nt)
     return fail(XF_ERR_INVALID, "not enough time-table steps left to tune");
-  XF_TRY(snapshot());
+  int status = snapshot();
+  if (status == XF_ERR_NOMEM && step3_ready) {  // no room for both
+    SecondSets::all().remove(this);
+    give_back();
+    status = snapshot();
+  }
+  if (status != XF_OK) return status;
   const int64_t step0 = cur_step;
   const xf_timing keep = timing;
   const int keep_timing = plan.timing;
   plan.timing = 0;
   xf_tuning win{};
   win.step_ms = 1e30;
-  int status = XF_OK;
   const std::vector<int> tys = dim == 3 ? std::vector<int>{1, 2, 4} : std::vector<int>{1};
   const std::vector<int> pls = dim == 3 ? std::vector<int>{2, 4, 8, 16} : std::vector<int>{1};
   // the z-face split and tail only where they change the launches
@@ -968,6 +1006,7 @@ int Engine::autotune(int trial_steps, xf_tuning* best) {
     set_tiling(0, 0, 0);
     return XF_OK;
   }
+  SecondSets::all().remove(this);
   step3_drop();
   set_tiling(win.tile_y, static_cast<int>((nx + 1 + win.planes - 1) / win.planes),
              XF_TILE_SET | (win.nontemporal ? XF_TILE_NT : 0) | (win.pml_split == 1 ? XF_TILE_PML_SPLIT : 0) |
@@ -987,6 +1026,7 @@ int xf_autotune(xf_handle* h, int32_t trial_steps, xf_tuning* best) {
   return xf::guarded([&]() -> int {
     xf::g_err.clear();
     if (!h) return xf::fail(XF_ERR_INVALID, "null handle");
+    std::lock_guard<std::mutex> work(h->eng.busy);
     return h->eng.autotune(trial_steps, best);
   });
 }
@@ -1009,6 +1049,7 @@ int xf_batch_upload(xf_batch* b) {
   return xf::guarded([&]() -> int {
     xf::g_err.clear();
     if (!b) return xf::fail(XF_ERR_INVALID, "null batch");
+    std::lock_guard<std::mutex> work(b->b.busy);
     const int st = xf::guarded([&] { return b->b.upload(); });
     if (st != XF_OK) b->b.release();
     return st;
@@ -1019,6 +1060,7 @@ int xf_batch_run(xf_batch* b, int64_t n_steps) {
   return xf::guarded([&]() -> int {
     xf::g_err.clear();
     if (!b) return xf::fail(XF_ERR_INVALID, "null batch");
+    std::lock_guard<std::mutex> work(b->b.busy);
     return b->b.run(n_steps);
   });
 }
@@ -1027,6 +1069,7 @@ int xf_batch_download(xf_batch* b) {
   return xf::guarded([&]() -> int {
     xf::g_err.clear();
     if (!b) return xf::fail(XF_ERR_INVALID, "null batch");
+    std::lock_guard<std::mutex> work(b->b.busy);
     return b->b.download();
   });
 }
@@ -1042,6 +1085,7 @@ int xf_batch_set_tuning(xf_batch* b, const xf_tuning* t) {
   return xf::guarded([&]() -> int {
     xf::g_err.clear();
     if (!b || !t) return xf::fail(XF_ERR_INVALID, "null argument");
+    std::lock_guard<std::mutex> work(b->b.busy);
     const xf_tuning keep = b->b.tune;
     const bool keep_auto = b->b.step3_auto;
     b->b.tune = *t;
@@ -1076,6 +1120,7 @@ int xf_batch_autotune(xf_batch* b, int32_t trial_steps, xf_tuning* best) {
   return xf::guarded([&]() -> int {
     xf::g_err.clear();
     if (!b) return xf::fail(XF_ERR_INVALID, "null batch");
+    std::lock_guard<std::mutex> work(b->b.busy);
     return b->b.autotune(trial_steps, best);
   });
 }
@@ -1107,6 +1152,7 @@ int xf_batch_set_timing(xf_batch* b, int32_t on) {
 int xf_batch_describe(const xf_batch* b, char* buf, size_t len) {
   return xf::guarded([&]() -> int {
     if (!b || !buf || len == 0) return xf::fail(XF_ERR_INVALID, "null argument");
+    std::lock_guard<std::mutex> lock(b->b.desc_m);
     std::snprintf(buf, len, "%s", b->b.desc.c_str());
     return XF_OK;
   });

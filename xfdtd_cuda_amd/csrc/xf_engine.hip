@@ -7,6 +7,8 @@
 #include <algorithm>
 #include <numeric>
 #include <array>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -17,6 +19,7 @@
 #include <stdexcept>
 #include <string>
 #include <system_error>
+#include <mutex>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -147,8 +150,89 @@ struct TfsfJobHost {
 
 }  // namespace
 
+// ------------------------------------------------------------ second sets
+// An engine or a batch that holds the one-pass step's second set of fields.
+struct SecondSet {
+  std::mutex busy;                   // held by the call that works on the handle
+  std::atomic<bool> waiting{false};  // ... while it waits for another's set
+  virtual void give_back() = 0;
+
+ protected:
+  ~SecondSet() = default;
+};
+
+// The process's holders.  A device allocation that fails is tried again after
+// another holder on that device has given its set back (it steps in two passes
+// from then on, with the same results): what fits the device without second
+// sets is never refused because of them.  A holder in the middle of a call is
+// waited for.
+class SecondSets {
+ public:
+  static SecondSets& all() {
+    static SecondSets* s = new SecondSets;  // outlives every handle
+    return *s;
+  }
+  void add(SecondSet* s, int device, size_t bytes) {
+    std::lock_guard<std::mutex> lock(m_);
+    held_.push_back({s, device, bytes});
+  }
+  void remove(const SecondSet* s) {
+    std::lock_guard<std::mutex> lock(m_);
+    held_.erase(std::remove_if(held_.begin(), held_.end(), [&](const Held& h) { return h.set == s; }), held_.end());
+  }
+  // hipMalloc for a call that works on `self` (whose own set is its own
+  // matter), or for none that has one
+  hipError_t malloc(void** p, size_t bytes, int device, SecondSet* self) {
+    hipError_t e = hipMalloc(p, bytes);
+    while (e != hipSuccess) {
+      (void)hipGetLastError();
+      *p = nullptr;
+      const Got got = take_back(bytes, device, self);
+      if (got == Got::none) break;
+      if (got == Got::later) {
+        if (self) self->waiting = true;  // two that wait for each other do not wait on
+        std::this_thread::sleep_for(std::chrono::milliseconds(1));
+      }
+      e = hipMalloc(p, bytes);
+    }
+    if (self) self->waiting = false;
+    return e;
+  }
+
+ private:
+  struct Held {
+    SecondSet* set;
+    int device;
+    size_t bytes;
+  };
+  enum class Got { one, later, none };
+  Got take_back(size_t bytes, int device, const SecondSet* self) {
+    std::lock_guard<std::mutex> lock(m_);
+    size_t room = 0, all = 0;
+    if (hipMemGetInfo(&room, &all) != hipSuccess) return Got::none;
+    for (const Held& h : held_)
+      if (h.device == device && h.set != self) room += h.bytes;
+    if (room < bytes) return Got::none;  // not for what cannot fit anyway
+    Got got = Got::none;
+    for (size_t q = held_.size(); q-- > 0;) {
+      SecondSet* const s = held_[q].set;
+      if (held_[q].device != device || s == self) continue;
+      const std::unique_lock<std::mutex> idle(s->busy, std::try_to_lock);
+      if (idle.owns_lock()) {
+        s->give_back();
+        held_.erase(held_.begin() + static_cast<std::ptrdiff_t>(q));
+        return Got::one;
+      }
+      if (!s->waiting) got = Got::later;
+    }
+    return got;
+  }
+  std::mutex m_;
+  std::vector<Held> held_;
+};
+
 // ---------------------------------------------------------------- engine
-struct Engine {
+struct Engine : SecondSet {
   xf_scene* sc{};
   xf_plan plan{};
   int dim{3};
@@ -173,10 +257,10 @@ struct Engine {
   // counts the swaps modulo two: the descriptor a launch takes.
   void* fld2[6]{};
   bool step3_form{false};   // the scene has the one-pass form
-  bool step3_ready{false};  // ... and its tables and the second set are on the device
+  std::atomic<bool> step3_ready{false};  // ... and its tables and the second set are on the device
   bool step3_auto{true};    // the tiling was left to the engine
   int step3_set{0};
-  bool in_batch{false};     // the batch decides on the second set
+  SecondSet* batch{};       // the batch the engine is in: it decides on the second set
   std::vector<uint8_t> step3_ids_h;  // one byte per node: row of step3_tab
   std::vector<double> step3_tab_h;   // 18 coefficients per pair of E and H rows
   void* step3_ids{};
@@ -218,6 +302,7 @@ struct Engine {
   void step3_drop();
   void step3_forget();
   void step3_settle();
+  void give_back() override;
   template <typename S>
   Step3Pass<S> step3_pass() const;
   template <typename S>
@@ -338,6 +423,7 @@ struct Engine {
   Tiling tiling() const;
   int snapshot();  // copy every state buffer aside (device to device)
   int restore();   // put the copies back; the step counter is the caller's
+  void drop_backup();
   int autotune(int trial_steps, xf_tuning* best);
   template <typename S>
   YeePass<S> yee_pass(bool is_e) const;
@@ -350,10 +436,12 @@ struct Engine {
     return d;
   }
   std::string layout_desc;
+  mutable std::mutex layout_m;  // layout_desc: another handle's call may have the set given back
 
   ~Engine() { release(); }
 
   void release() {
+    if (!batch) SecondSets::all().remove(this);
     drop_graph();
     for (void* p : allocs) (void)hipFree(p);
     allocs.clear();
@@ -381,7 +469,7 @@ struct Engine {
   int alloc(void** p, size_t bytes) {
     *p = nullptr;
     if (bytes == 0) bytes = 16;
-    hipError_t e = hipMalloc(p, bytes);
+    hipError_t e = SecondSets::all().malloc(p, bytes, device, batch ? batch : this);
     if (e != hipSuccess) return fail(XF_ERR_NOMEM, "hipMalloc(" + std::to_string(bytes) + "): " + hipGetErrorString(e));
     allocs.push_back(*p);
     return XF_OK;
@@ -1434,7 +1522,7 @@ bool Engine::step3_take() {
        hipMemcpyHostToDevice);
   ok = ok && hipStreamSynchronize(stream) == hipSuccess;
   step3_set = 0;
-  if (ok && !in_batch) {  // a batch has descriptors of its own
+  if (ok && !batch) {  // a batch has descriptors of its own
     void* start = nullptr;
     take(&step3_desc, 2 * sizeof(Step3Pass<double>));
     take(&start, 2 * sizeof(int));
@@ -1486,15 +1574,21 @@ void Engine::step3_drop() {
 // engine and the set takes at most a quarter of the device memory that is
 // free (the rest is left to other engines and to the caller).
 void Engine::step3_settle() {
-  if (in_batch || !stream) return;
+  if (batch || !stream) return;
   if (!step3_auto) {
+    SecondSets::all().remove(this);
     step3_drop();
   } else if (step3_form && !step3_ready) {
     size_t free_bytes = 0, all_bytes = 0;
     if (hipSetDevice(device) == hipSuccess && hipMemGetInfo(&free_bytes, &all_bytes) == hipSuccess &&
-        step3_bytes() <= free_bytes / 4)
-      (void)step3_take();
+        step3_bytes() <= free_bytes / 4 && step3_take())
+      SecondSets::all().add(this, device, step3_bytes());
   }
+  describe_layout();
+}
+
+void Engine::give_back() {
+  step3_drop();
   describe_layout();
 }
 
@@ -2142,7 +2236,7 @@ void Engine::set_tiling(int ty, int chunks_x, int flags) {
 }
 
 void Engine::describe_layout() {
-  layout_desc = std::string("dim=") + std::to_string(dim) + " pad_stride=" + std::to_string(dim == 3 ? sy : sx) +
+  const std::string desc = std::string("dim=") + std::to_string(dim) + " pad_stride=" + std::to_string(dim == 3 ? sy : sx) +
                 " id_bytes=" + std::to_string(id_bytes) + " coeff=" + (dense ? "dense" : "table") +
                 " etab=" + std::to_string(ntab_e) +
                 " htab=" + std::to_string(ntab_h) + " chunk=" + std::to_string(chunk) +
@@ -2156,6 +2250,17 @@ void Engine::describe_layout() {
                 " step3=" + std::to_string(use_step3() ? 1 : 0) +
                 (use_step3() ? " step3_chunk=" + std::to_string(step3_chunk) + " step3_rows=" + std::to_string(step3_rows)
                              : std::string());
+  std::lock_guard<std::mutex> lock(layout_m);
+  layout_desc = desc;
+}
+
+void Engine::drop_backup() {
+  for (void* p : backup)
+    if (p) {
+      (void)hipFree(p);
+      allocs.erase(std::find(allocs.begin(), allocs.end(), p));
+    }
+  backup.clear();
 }
 
 int Engine::snapshot() {
@@ -2163,7 +2268,12 @@ int Engine::snapshot() {
   XF_HIP(hipSetDevice(device));
   if (backup.size() != state.size()) {
     backup.assign(state.size(), nullptr);
-    for (size_t q = 0; q < state.size(); ++q) XF_TRY(alloc(&backup[q], state[q].second));
+    for (size_t q = 0; q < state.size(); ++q) {
+      const int st = alloc(&backup[q], state[q].second);
+      if (st == XF_OK) continue;
+      drop_backup();
+      return st;
+    }
   }
   for (size_t q = 0; q < state.size(); ++q)
     XF_HIP(hipMemcpyAsync(backup[q], live(state[q].first), state[q].second, hipMemcpyDeviceToDevice, stream));
@@ -3329,6 +3439,7 @@ int xf_upload(xf_handle* h) {
     int n = 0;
     if (hipGetDeviceCount(&n) != hipSuccess || n == 0) return xf::fail(XF_ERR_HIP, "no HIP device");
     if (h->eng.device < 0 || h->eng.device >= n) return xf::fail(XF_ERR_INVALID, "bad device ordinal");
+    std::lock_guard<std::mutex> work(h->eng.busy);
     // a failed upload (status or exception) leaves nothing on the device
     const int st = xf::guarded([&] { return h->eng.upload(); });
     if (st != XF_OK) h->eng.release();
@@ -3340,6 +3451,7 @@ int xf_run(xf_handle* h, int64_t n_steps) {
   return xf::guarded([&]() -> int {
     xf::g_err.clear();
     if (!h) return xf::fail(XF_ERR_INVALID, "null handle");
+    std::lock_guard<std::mutex> work(h->eng.busy);
     return h->eng.run(n_steps);
   });
 }
@@ -3348,6 +3460,7 @@ int xf_download(xf_handle* h) {
   return xf::guarded([&]() -> int {
     xf::g_err.clear();
     if (!h) return xf::fail(XF_ERR_INVALID, "null handle");
+    std::lock_guard<std::mutex> work(h->eng.busy);
     return h->eng.download();
   });
 }
@@ -3393,8 +3506,11 @@ int xf_stream_bench(int64_t bytes, int32_t reps, int32_t device, int32_t variant
     if (hipSetDevice(device) != hipSuccess) return xf::fail(XF_ERR_HIP, "hipSetDevice failed");
     const int64_t n = bytes / 16;
     xf::xf_d2 *a = nullptr, *b = nullptr;
-    if (hipMalloc(&a, n * 16) != hipSuccess) return xf::fail(XF_ERR_NOMEM, "stream bench allocation failed");
-    if (hipMalloc(&b, n * 16) != hipSuccess) {
+    auto take = [&](xf::xf_d2** p) {
+      return xf::SecondSets::all().malloc(reinterpret_cast<void**>(p), n * 16, device, nullptr) == hipSuccess;
+    };
+    if (!take(&a)) return xf::fail(XF_ERR_NOMEM, "stream bench allocation failed");
+    if (!take(&b)) {
       (void)hipFree(a);
       return xf::fail(XF_ERR_NOMEM, "stream bench allocation failed");
     }
@@ -3436,6 +3552,7 @@ int xf_set_tiling(xf_handle* h, int32_t tile_y, int32_t chunks_x, int32_t flags)
     if (!h) return xf::fail(XF_ERR_INVALID, "null handle");
     // the Yee kernels are compiled for at most 256 threads per block (64 x 4)
     if (tile_y < 0 || tile_y > 4 || chunks_x < 0) return xf::fail(XF_ERR_INVALID, "bad tiling (tile_y 0..4)");
+    std::lock_guard<std::mutex> work(h->eng.busy);
     h->eng.set_tiling(tile_y, chunks_x, flags);
     h->eng.step3_settle();
     return XF_OK;
@@ -3453,6 +3570,7 @@ int xf_set_timing(xf_handle* h, int32_t on) {
 int xf_describe(const xf_handle* h, char* buf, size_t len) {
   return xf::guarded([&]() -> int {
     if (!h || !buf || len == 0) return xf::fail(XF_ERR_INVALID, "null argument");
+    std::lock_guard<std::mutex> lock(h->eng.layout_m);
     std::snprintf(buf, len, "%s", h->eng.layout_desc.c_str());
     return XF_OK;
   });

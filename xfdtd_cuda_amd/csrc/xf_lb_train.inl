@@ -413,7 +413,7 @@ struct LbTrainer {
 
   int alloc(void** p, size_t bytes) {
     *p = nullptr;
-    hipError_t e = hipMalloc(p, bytes ? bytes : 16);
+    hipError_t e = SecondSets::all().malloc(p, bytes ? bytes : 16, device, nullptr);
     if (e != hipSuccess) return fail(XF_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     allocs.push_back(*p);
     return XF_OK;
