@@ -848,6 +848,7 @@ int Batch::autotune(int trial_steps, xf_tuning* best) {
     h->eng.pml_ztail = keep_tail;
   }
   // the one-pass step, then the two-pass tilings
+  const xf_tuning keep_tune = tune;
   const bool keep_auto = step3_auto;
   bool win_step3 = false;
   step3_auto = true;
@@ -908,12 +909,15 @@ int Batch::autotune(int trial_steps, xf_tuning* best) {
   cur_step = step0;
   sync_steps();
   step3_auto = status == XF_OK ? win_step3 : keep_auto;
+  tune = status == XF_OK ? win : keep_tune;
+  if (!step3_auto) drop_sets();
   if (status != XF_OK) {
+    // as it was: descriptors, graphs and sets of the tuning before, and the state
+    const std::string why = g_err;
+    stale = configure() != XF_OK;
     (void)restore();
-    return status;
+    return fail(status, why);
   }
-  tune = win;
-  if (!win_step3) drop_sets();
   XF_TRY(configure());
   if (best) *best = win;
   return XF_OK;
@@ -934,6 +938,7 @@ int Engine::autotune(int trial_steps, xf_tuning* best) {
   if (status != XF_OK) return status;
   const int64_t step0 = cur_step;
   const xf_timing keep = timing;
+  const xf_plan keep_plan = plan;
   const int keep_timing = plan.timing;
   plan.timing = 0;
   xf_tuning win{};
@@ -998,8 +1003,11 @@ int Engine::autotune(int trial_steps, xf_tuning* best) {
   timing = keep;
   cur_step = step0;
   if (status != XF_OK) {
+    const std::string why = g_err;
+    set_tiling(keep_plan.tile_y, keep_plan.chunks_x, keep_plan.tiling_flags);
+    step3_settle();
     (void)restore();
-    return status;
+    return fail(status, why);
   }
   if (best) *best = win;
   if (win_step3) {
