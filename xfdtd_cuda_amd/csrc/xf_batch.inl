@@ -780,6 +780,7 @@ int Batch::run(int64_t n) {
 
 int Batch::download() {
   if (!uploaded) return fail(XF_ERR_STATE, "download before upload");
+  XF_HIP(hipSetDevice(device));
   XF_HIP(hipStreamSynchronize(stream));
   if (inst.empty()) return XF_OK;
   // one pass through the staging slots for every grid

@@ -2305,6 +2305,7 @@ Tiling Engine::tiling() const {
 // ------------------------------------------------------------- download
 int Engine::download() {
   if (!uploaded) return fail(XF_ERR_STATE, "download before upload");
+  XF_HIP(hipSetDevice(device));  // the slots' events belong to the stream's device
   XF_HIP(hipStreamSynchronize(stream));
   {
     Drain out(stages, stream, plane_bytes(), drain_bytes());
