@@ -302,8 +302,9 @@ typedef struct xf_plan {
   int32_t chunks_x;     /* 0 = auto; x-chunks of the 3-D marching kernels */
   int32_t tiling_flags; /* 0 = auto, else XF_TILE_SET | XF_TILE_* bits.  With
                            tile_y, chunks_x and these at 0 a 3-D step runs H and
-                           E in one pass where the scene allows it; a tiling
-                           given by hand takes the two-pass kernels           */
+                           E in one pass where the scene allows it and the
+                           grid's shape favours it; a tiling given by hand takes
+                           the two-pass kernels                               */
   int32_t coeff_mode;   /* enum xf_coeff_mode                              */
   int32_t watchdog;     /* 0 = off; else every `watchdog` steps (and after
                            the last step of each xf_run) every stored field

@@ -62,7 +62,10 @@ struct Batch : SecondSet {
   bool lb_any_record{false};
   int* t_dev{};
   // the one-pass step of every grid in one launch (each grid's blocks in turn)
-  bool step3_auto{true};  // the tiling was left to the engine
+  bool step3_won{false};  // as Engine's
+  bool step3_pick{true};
+  bool step3_auto{true};  // the tuning was left to the engine
+  bool step3_pays();
   void* step3_desc{};     // [2][grids] Step3Pass
   int* step3_start{};
   int step3_blocks{0};
@@ -212,6 +215,7 @@ int Batch::upload() {
   void* tp;
   XF_TRY(alloc(&tp, sizeof(int)));
   t_dev = static_cast<int*>(tp);
+  step3_pick = step3_won || step3_pays();
   XF_TRY(configure());
   uploaded = true;
   return XF_OK;
@@ -236,6 +240,23 @@ bool Batch::take_sets() {
   else
     for (auto& h : inst) h->eng.step3_drop();
   return all;
+}
+
+// Where one pass is the faster step (Engine::step3_pays for a grid alone; a
+// batch's two passes have other tiles).  FP32 blocks whose CPML waves meet both
+// ends of z are slower: 16 grids of 113 x 113 x 65 nodes 693 / 577 us a step,
+// 8 of 213 x 213 x 33 631 / 540; in FP64 both are even (952 / 941, 836 / 883),
+// in 16 bits faster (697 / 1052, 636 / 946).
+bool Batch::step3_pays() {
+  if (plan.precision != XF_FP32) return true;
+  double rounds = 0, slow = 0;
+  for (auto& h : inst) {
+    const Engine& E = h->eng;
+    const double r = E.step3_rounds();
+    rounds += r;
+    if (!E.pml.empty() && (E.nz >= 64 || E.nz < 48 || E.sc->tfsf) && E.step3_both_ends(true)) slow += r;
+  }
+  return rounds < 20 || 2 * slow < rounds;
 }
 
 // The grids' descriptors are to be made again (configure) after it.
@@ -524,7 +545,7 @@ int Batch::configure() {
   if (tune.blocks < 0) return fail(XF_ERR_INVALID, "blocks must be >= 0");
   XF_HIP(hipSetDevice(device));
   drop_graph();
-  if (step3_auto) (void)take_sets();
+  if (step3_auto && step3_pick) (void)take_sets();
   int st;
   switch (plan.precision) {
     case XF_FP64: st = configure_t<double>(); break;
@@ -910,8 +931,9 @@ int Batch::autotune(int trial_steps, xf_tuning* best) {
   cur_step = step0;
   sync_steps();
   step3_auto = status == XF_OK ? win_step3 : keep_auto;
+  if (status == XF_OK) step3_won = step3_pick = win_step3;
   tune = status == XF_OK ? win : keep_tune;
-  if (!step3_auto) drop_sets();
+  if (!step3_auto || !step3_pick) drop_sets();
   if (status != XF_OK) {
     // as it was: descriptors, graphs and sets of the tuning before, and the state
     const std::string why = g_err;
@@ -957,7 +979,9 @@ int Engine::autotune(int trial_steps, xf_tuning* best) {
   pml_ztail = keep_tail;
   // the one-pass step, then the two-pass tilings
   bool win_step3 = false;
+  const bool keep_pick = step3_pick;
   if (step3_form) {
+    step3_pick = true;
     set_tiling(0, 0, 0);
     step3_settle();
   }
@@ -1005,16 +1029,19 @@ int Engine::autotune(int trial_steps, xf_tuning* best) {
   cur_step = step0;
   if (status != XF_OK) {
     const std::string why = g_err;
+    step3_pick = keep_pick;
     set_tiling(keep_plan.tile_y, keep_plan.chunks_x, keep_plan.tiling_flags);
     step3_settle();
     (void)restore();
     return fail(status, why);
   }
   if (best) *best = win;
+  step3_won = win_step3;
   if (win_step3) {
     set_tiling(0, 0, 0);
     return XF_OK;
   }
+  step3_pick = keep_pick;
   SecondSets::all().remove(this);
   step3_drop();
   set_tiling(win.tile_y, static_cast<int>((nx + 1 + win.planes - 1) / win.planes),

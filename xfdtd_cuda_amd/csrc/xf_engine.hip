@@ -258,7 +258,9 @@ struct Engine : SecondSet {
   void* fld2[6]{};
   bool step3_form{false};   // the scene has the one-pass form
   std::atomic<bool> step3_ready{false};  // ... and its tables and the second set are on the device
-  bool step3_auto{true};    // the tiling was left to the engine
+  bool step3_won{false};    // the tuner found it the faster one
+  bool step3_pick{true};    // ... or step3_pays expects so
+  bool step3_auto{true};    // the tiling was left to the engine, which picks it
   int step3_set{0};
   SecondSet* batch{};       // the batch the engine is in: it decides on the second set
   std::vector<uint8_t> step3_ids_h;  // one byte per node: row of step3_tab
@@ -270,10 +272,8 @@ struct Engine : SecondSet {
   void* step3_desc{};       // two Step3Pass, one per direction
   int* step3_start{};
   int step3_blocks{0}, step3_chunk{1};
-  // One pass wherever the scene has the form (step3_tables, step3_incident,
-  // step3_faces): on the grids measured it is the faster one or even, us a
-  // step against two passes: 536^3 FP64 3765 / 4730, 148^3 FP64 167 / 204,
-  // 253^3 FP32 414 / 419, FP16 storage 419 / 483.
+  // One pass where the scene has the form (step3_tables, step3_incident,
+  // step3_faces) and it pays (step3_pays).
   bool use_step3() const { return step3_ready && step3_auto; }
   void step3_swap() {
     std::swap_ranges(fld, fld + 6, fld2);
@@ -296,6 +296,9 @@ struct Engine : SecondSet {
   bool step3_incident() const;
   template <typename C>
   bool step3_faces() const;
+  double step3_rounds() const;
+  bool step3_both_ends(bool tfsf) const;
+  bool step3_pays() const;
   size_t step3_psi_bytes(size_t q, int c) const;
   size_t step3_bytes() const;
   bool step3_take();
@@ -2172,6 +2175,7 @@ int Engine::upload() {
   wd_dev = static_cast<unsigned*>(tp);
   step3_form = step3_rows > 0 && step3_incident() &&
                (plan.precision == XF_FP64 ? step3_faces<double>() : step3_faces<float>());
+  step3_pick = step3_won || step3_pays();
   set_tiling(plan.tile_y, plan.chunks_x, plan.tiling_flags);
   step3_settle();
   XF_HIP(hipDeviceSynchronize());
@@ -2190,7 +2194,7 @@ void Engine::set_tiling(int ty, int chunks_x, int flags) {
   plan.tile_y = ty;
   plan.chunks_x = chunks_x;
   plan.tiling_flags = flags;
-  step3_auto = ty == 0 && chunks_x == 0 && !(flags & XF_TILE_SET);
+  step3_auto = step3_pick && ty == 0 && chunks_x == 0 && !(flags & XF_TILE_SET);
   // 64 x tile_y threads must fit the kernels' __launch_bounds__(256)
   tile_y = ty > 0 ? std::min(ty, 4) : 1;
   if (flags & XF_TILE_SET) {
@@ -3078,6 +3082,70 @@ bool Engine::step3_faces() const {
     }
   }
   return true;
+}
+
+// Planes of k_step3's blocks for two blocks a CU: the time of a step in plane
+// times, once a launch fills the device.
+double Engine::step3_rounds() const {
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) cus = 256;
+  const int64_t planes = ((nz + 64) / 64) * ((ny + kStep3Rows) / kStep3Rows) * (nx + 1);
+  return static_cast<double>(planes) / (2.0 * std::max(1, cus));
+}
+
+// Whether a k tile of k_step3 meets the CPML (or a z face of the TF/SF box) at
+// both ends of the grid.
+bool Engine::step3_both_ends(bool tfsf) const {
+  int64_t low = -1, high = nz + 1;
+  PmlPass<double> P{};
+  fill_pml_pass<double>(*this, P, true);
+  for (int q = 0; q < P.n; ++q) {
+    const PmlFace<double>& F = P.f[q];
+    if (F.axis != 2) continue;
+    if (2 * F.c0 > nz)
+      high = std::min<int64_t>(high, F.c0);
+    else
+      low = std::max<int64_t>(low, F.c1 - 1);
+  }
+  if (tfsf && sc->tfsf) {
+    low = std::max<int64_t>(low, sc->tfsf->total_task.z.start);
+    high = std::min<int64_t>(high, sc->tfsf->total_task.z.end);
+  }
+  return low >= 0 && high <= nz && low / 64 * 64 + 63 >= high;
+}
+
+// Where one pass is the faster step.  On most grids it is (us a step against
+// two passes: 536^3 FP64 3765 / 4730, 148^3 FP64 167 / 204, 40^3 with CPML and
+// TF/SF 28 / 55), but its 64 lanes by six rows idle, and the marches of its
+// waves grow longer, where
+// - the grid is a few nodes wide across x or y: 901 x 901 x 2 nodes along z, y,
+//   x, FP64 45 / 28 (thin x) and 61 / 34 (thin y), FP32 28 / 18 and 38 / 18;
+// - FP64 has at most 32 nodes along z, one 32-lane tile of the two-pass
+//   kernels: 401 x 401 x 9 118 / 92, 409 x 409 x 17 with CPML 355 / 282
+//   (at 33 nodes, two tiles, 383 / 569);
+// - CPML waves meet both ends of z (a correction's chain twice a plane), in
+//   FP64 with a second tile beside them (409 x 409 x 65 718 / 487, 53 nodes
+//   412 / 478), in FP32 already in a single one that is not full or has the
+//   TF/SF faces (33 nodes 276 / 216, 53 with TF/SF 386 / 322), in 16 bits, whose
+//   two-pass CPML is slower, on large grids with TF/SF (741 / 577);
+// - narrow storage has TF/SF but no CPML: 225^3 FP16 180 / 138, compensated
+//   bf16 278 / 239 (161^3 FP16 73 / 72).
+// Below the rounds given it is the launches that count, and one is fewer:
+// 109 x 109 x 17 with CPML FP64 41 / 46, 209 x 209 x 33 FP32 82 / 90.
+bool Engine::step3_pays() const {
+  const double rounds = step3_rounds();
+  const int64_t ni = nx + 1, nj = ny + 1, nk = nz + 1;
+  const int64_t kb = (nk + 63) / 64, jb = (nj + kStep3Rows - 1) / kStep3Rows;
+  const bool f64 = esize == 8, f32 = esize == 4;
+  if (pml.empty()) {
+    if (ni <= 4 && rounds >= (f64 ? 1.5 : 6)) return false;
+    if (5 * nj < 3 * kStep3Rows * jb && rounds >= (f64 ? 1.5 : f32 ? 6 : 20)) return false;
+    if (esize < 4 && sc->tfsf && rounds >= 20) return false;
+  }
+  if (f64) return rounds < 6 || !(nk <= 32 || (kb > 1 && step3_both_ends(false)));
+  if (pml.empty()) return true;
+  if (f32) return rounds < 20 || !((kb > 1 || nk <= 48 || sc->tfsf) && step3_both_ends(true));
+  return esize == 3 || rounds < 50 || !(sc->tfsf && kb > 1 && step3_both_ends(true));
 }
 
 // Planes per chunk of k_step3 for the grids that share a launch.  A block
