@@ -436,14 +436,21 @@ int xf_stream_bench(int64_t bytes, int32_t reps, int32_t device, int32_t variant
 /* Tile shape of the 3-D Yee kernels, as set by hand or picked by an
  * autotuner (no reference counterpart: the reference takes the user's
  * grid/block dims, SimulationHD::setGridDim/setBlockDim,
- * simulation_hd.cuh:51-55, and decomposes flat index ranges). */
+ * simulation_hd.cuh:51-55, and decomposes flat index ranges).  The tuning an
+ * autotuner returns, or xf_batch_get_tuning of a batch on the device, given to
+ * xf_batch_set_tuning of this batch or another selects the same step again. */
+#define XF_TUNE_ONE_PASS 3
 typedef struct xf_tuning {
   int32_t tile_y;      /* 1..4: a block is 64 x tile_y threads (k32: 32 k-lanes x 2 tile_y rows) */
   int32_t planes;      /* x planes one block marches through (>= 1)        */
   int32_t blocks;      /* batch only: persistent grid size, 0 = resident   */
   int32_t nontemporal; /* stream the updated component non-temporally      */
   int32_t xcd_remap;   /* XCD-aware block order (batch: each XCD takes a contiguous eighth of the tiles) */
-  int32_t pml_split;   /* 0 z faces in the march, 1 XF_TILE_PML_SPLIT, 2 XF_TILE_PML_ZTAIL */
+  int32_t pml_split;   /* 0 z faces in the march, 1 XF_TILE_PML_SPLIT, 2 XF_TILE_PML_ZTAIL,
+                          3 (XF_TUNE_ONE_PASS) the one-pass step, which takes none of the
+                          other fields; two passes with them and split z faces where a
+                          scene lacks its form or the device the memory.  An engine is
+                          set to it by xf_set_tiling(h, 0, 0, 0) */
   int32_t k32;         /* XF_TILE_K32                                      */
   double step_ms;      /* autotune: measured time of one step              */
 } xf_tuning;

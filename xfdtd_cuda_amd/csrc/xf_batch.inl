@@ -317,7 +317,9 @@ int Batch::configure_t() {
   std::vector<int> ts(n + 1, 0);
   int64_t tiles = 0;
   pml_level = 0;
-  const int flags = XF_TILE_SET | (tune.nontemporal ? XF_TILE_NT : 0) | (tune.pml_split == 1 ? XF_TILE_PML_SPLIT : 0) |
+  // (XF_TUNE_ONE_PASS: the two passes in its place split the z faces off)
+  const int flags = XF_TILE_SET | (tune.nontemporal ? XF_TILE_NT : 0) |
+                    (tune.pml_split == 1 || tune.pml_split == XF_TUNE_ONE_PASS ? XF_TILE_PML_SPLIT : 0) |
                     (tune.pml_split == 2 ? XF_TILE_PML_ZTAIL : 0) | (tune.k32 ? XF_TILE_K32 : 0);
   for (int g = 0; g < n; ++g) {
     Engine& E = eng(g);
@@ -875,7 +877,7 @@ int Batch::autotune(int trial_steps, xf_tuning* best) {
   bool win_step3 = false;
   step3_auto = true;
   if (take_sets()) {
-    tune = xf_tuning{1, 4, 0, 1, 0, 1, 0, 0.0};
+    tune = xf_tuning{1, 4, 0, 1, 0, XF_TUNE_ONE_PASS, 0, 0.0};
     status = configure();
     if (status == XF_OK) status = run(1);
     if (status == XF_OK) status = run(trial_steps);
@@ -989,7 +991,7 @@ int Engine::autotune(int trial_steps, xf_tuning* best) {
     status = run(1);
     if (status == XF_OK) status = run(trial_steps);
     if (status == XF_OK) {
-      win = xf_tuning{1, step3_chunk, 0, 1, 0, 0, 0, timing.run_ms / trial_steps};
+      win = xf_tuning{1, step3_chunk, 0, 1, 0, XF_TUNE_ONE_PASS, 0, timing.run_ms / trial_steps};
       win_step3 = true;
       cur_step = step0;
       status = restore();
@@ -1123,21 +1125,23 @@ int xf_batch_set_tuning(xf_batch* b, const xf_tuning* t) {
     if (!b || !t) return xf::fail(XF_ERR_INVALID, "null argument");
     std::lock_guard<std::mutex> work(b->b.busy);
     const xf_tuning keep = b->b.tune;
-    const bool keep_auto = b->b.step3_auto;
+    if (t->tile_y < 1 || t->tile_y > 4 || t->planes < 1 || t->blocks < 0 || t->pml_split < 0 ||
+        t->pml_split > XF_TUNE_ONE_PASS)
+      return xf::fail(XF_ERR_INVALID, "bad tuning (tile_y 1..4, planes >= 1, blocks >= 0, pml_split 0..3)");
+    const bool keep_auto = b->b.step3_auto, keep_won = b->b.step3_won, keep_pick = b->b.step3_pick;
+    const bool one_pass = t->pml_split == XF_TUNE_ONE_PASS;
     b->b.tune = *t;
     b->b.tune.step_ms = 0;
-    b->b.step3_auto = false;
-    if (t->tile_y < 1 || t->tile_y > 4 || t->planes < 1 || t->blocks < 0 || t->pml_split < 0 || t->pml_split > 2) {
-      b->b.tune = keep;
-      b->b.step3_auto = keep_auto;
-      return xf::fail(XF_ERR_INVALID, "bad tuning (tile_y 1..4, planes >= 1, blocks >= 0, pml_split 0..2)");
-    }
+    b->b.step3_auto = b->b.step3_won = one_pass;
+    if (one_pass) b->b.step3_pick = true;
     if (!b->b.uploaded) return XF_OK;
-    b->b.drop_sets();
+    if (!one_pass) b->b.drop_sets();
     const int st = b->b.configure();
     if (st != XF_OK) {
       b->b.tune = keep;
       b->b.step3_auto = keep_auto;
+      b->b.step3_won = keep_won;
+      b->b.step3_pick = keep_pick;
       (void)b->b.configure();
     }
     return st;
@@ -1148,6 +1152,11 @@ int xf_batch_get_tuning(const xf_batch* b, xf_tuning* t) {
   return xf::guarded([&]() -> int {
     if (!b || !t) return xf::fail(XF_ERR_INVALID, "null argument");
     *t = b->b.tune;
+    // what runs: the one-pass step by the engine's own choice too, not where memory ruled it out
+    if (b->b.uploaded && b->b.use_step3())
+      t->pml_split = XF_TUNE_ONE_PASS;
+    else if (b->b.uploaded && t->pml_split == XF_TUNE_ONE_PASS)
+      t->pml_split = 1;
     return XF_OK;
   });
 }

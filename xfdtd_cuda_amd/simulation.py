@@ -539,7 +539,8 @@ class Engine:
 
     def autotune(self, trial_steps: int = 3) -> dict:
         """Times candidate tilings on this scene (state restored after each)
-        and keeps the fastest; returns it."""
+        and keeps the fastest; returns it (pml_split 3: the one-pass step,
+        which set_tiling() without arguments selects again)."""
         t = XfTuning()
         _native.check_hip(self._lib.xf_autotune(self._h, trial_steps, ctypes.byref(t)),
                           "xf_autotune")
@@ -597,8 +598,9 @@ class Batch:
                    nontemporal: bool = True, pml_split: bool = True, k32: bool = False,
                    xcd_remap: bool = False, pml_ztail: bool = False):
         """pml_split: z-face CPML in a launch of its own; pml_ztail (takes
-        precedence): at the end of each Yee tile."""
-        split = 2 if pml_ztail else int(bool(pml_split))
+        precedence): at the end of each Yee tile.  pml_split=3, as tuning()
+        and autotune() give it: the one-pass step."""
+        split = 2 if pml_ztail else 3 if pml_split == 3 else int(bool(pml_split))
         t = XfTuning(tile_y, planes, blocks, int(nontemporal), int(xcd_remap), split, int(k32), 0.0)
         _native.check_hip(self._lib.xf_batch_set_tuning(self._h, ctypes.byref(t)),
                           "xf_batch_set_tuning")
