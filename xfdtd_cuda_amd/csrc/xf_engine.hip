@@ -263,8 +263,8 @@ struct Engine : SecondSet {
   bool step3_auto{true};    // the tiling was left to the engine, which picks it
   int step3_set{0};
   SecondSet* batch{};       // the batch the engine is in: it decides on the second set
-  std::vector<uint8_t> step3_ids_h;  // one byte per node: row of step3_tab
-  std::vector<double> step3_tab_h;   // 18 coefficients per pair of E and H rows
+  std::unique_ptr<uint8_t[]> step3_ids_h;  // one byte per node: row of step3_tab
+  std::vector<double> step3_tab_h;         // 18 coefficients per pair of E and H rows
   void* step3_ids{};
   void* step3_tab{};
   int step3_rows{0};
@@ -453,7 +453,7 @@ struct Engine : SecondSet {
     std::fill(fld2, fld2 + 6, nullptr);
     step3_form = step3_ready = false;
     step3_set = 0;
-    step3_ids_h = {};
+    step3_ids_h.reset();
     step3_tab_h = {};
     step3_ids = step3_tab = step3_desc = nullptr;
     step3_start = nullptr;
@@ -1425,26 +1425,38 @@ void Engine::step3_tables(const std::vector<uint32_t>& ide, const std::vector<ui
   step3_rows = 0;
   if (dense || dim != 3 || sy >= (int64_t(1) << 24) || ntab_e > kStep3MaxRows || ntab_h > kStep3MaxRows) return;
   const size_t most = has_ade ? kStep3AdeRows : kStep3MaxRows;
-  std::vector<int> at(static_cast<size_t>(ntab_e) * ntab_h, -1);
-  std::vector<std::pair<int, int>> pairs{{0, 0}};
-  at[0] = 0;
-  const int64_t cells = nx * ny * nz;
-  int64_t run_end = 0;
-  uint32_t le = 0, lh = 0;
-  std::vector<uint8_t> id(static_cast<size_t>(cells));
-  for (int64_t c = 0; c < cells; ++c) {
-    if (c == 0 || ide[c] != le || idh[c] != lh) {
-      le = ide[c];
-      lh = idh[c];
-      int& p = at[static_cast<size_t>(le) * ntab_h + lh];
-      if (p < 0) {
-        if (pairs.size() >= most) return;
-        p = static_cast<int>(pairs.size());
-        pairs.emplace_back(static_cast<int>(le), static_cast<int>(lh));
+  // one thread takes some 100 ms for 536^3 cells (an upload of 1.7 s), and on
+  // smaller grids no longer than threads take to start
+  const auto planes = [&](int64_t n, auto fn) {
+    if (nx * ny * nz < (int64_t(1) << 23))
+      fn(int64_t(0), n);
+    else
+      host_parallel_for(n, fn);
+  };
+  // cells [c0, c1) in runs of one pair
+  const auto runs = [&](int64_t c0, int64_t c1, auto fn) {
+    for (int64_t c = c0, n; c < c1; c = n) {
+      const uint32_t e = ide[c], h = idh[c];
+      uint32_t other = 0;
+      for (n = c + 1; n + 8 <= c1; n += 8) {
+        for (int q = 0; q < 8; ++q) other |= (ide[n + q] ^ e) | (idh[n + q] ^ h);
+        if (other) break;
       }
-      run_end = p;
+      while (n < c1 && ide[n] == e && idh[n] == h) ++n;
+      fn(c, n, static_cast<size_t>(e) * ntab_h + h);
     }
-    id[c] = static_cast<uint8_t>(run_end);
+  };
+  std::vector<std::atomic<bool>> seen(static_cast<size_t>(ntab_e) * ntab_h);
+  planes(nx, [&](int64_t i0, int64_t i1) {
+    runs(i0 * ny * nz, i1 * ny * nz, [&](int64_t, int64_t, size_t p) { seen[p].store(true, std::memory_order_relaxed); });
+  });
+  std::vector<uint8_t> at(seen.size(), 0);
+  std::vector<std::pair<int, int>> pairs{{0, 0}};
+  for (size_t p = 1; p < seen.size(); ++p) {
+    if (!seen[p].load(std::memory_order_relaxed)) continue;
+    if (pairs.size() >= most) return;
+    at[p] = static_cast<uint8_t>(pairs.size());
+    pairs.emplace_back(static_cast<int>(p / ntab_h), static_cast<int>(p % ntab_h));
   }
   step3_dmask = 0;
   for (size_t q = 0; q < pairs.size(); ++q) {
@@ -1453,10 +1465,20 @@ void Engine::step3_tables(const std::vector<uint32_t>& ide, const std::vector<ui
     if (has_ade && eflag_h[pairs[q].first]) step3_dmask |= uint64_t(1) << q;
   }
   step3_rows = static_cast<int>(pairs.size());
-  step3_ids_h.assign(total, 0);
-  for (int64_t i = 0; i < nx; ++i)
-    for (int64_t j = 0; j < ny; ++j)
-      std::copy_n(id.data() + (i * ny + j) * nz, nz, step3_ids_h.data() + i * sx + j * sy);
+  step3_ids_h.reset(new uint8_t[static_cast<size_t>(total)]);
+  planes(nx + 1, [&](int64_t i0, int64_t i1) {
+    for (int64_t i = i0; i < i1; ++i) {
+      uint8_t* const to = step3_ids_h.get() + i * sx;
+      std::memset(to, 0, static_cast<size_t>(sx));
+      if (i == nx) continue;
+      for (int64_t j = 0; j < ny; ++j) {
+        const int64_t c = (i * ny + j) * nz;
+        runs(c, c + nz, [&](int64_t a, int64_t b, size_t p) {
+          std::memset(to + j * sy + (a - c), at[p], static_cast<size_t>(b - a));
+        });
+      }
+    }
+  });
 }
 
 // Whether a block's share of the incident tables is bounded as k_step3 holds
@@ -1514,12 +1536,12 @@ bool Engine::step3_take() {
   for (int c = 0; c < 6; ++c) take(&fld2[c], static_cast<size_t>(total) * esize);
   for (size_t q = 0; q < pml.size(); ++q)
     for (int c = 0; c < 2; ++c) take(&pml[q].psi2[c], step3_psi_bytes(q, c));
-  take(&step3_ids, step3_ids_h.size());
+  take(&step3_ids, static_cast<size_t>(total));
   take(&step3_tab, step3_lds());
   for (int c = 0; c < 6; ++c) copy(fld2[c], fld[c], static_cast<size_t>(total) * esize, hipMemcpyDeviceToDevice);
   for (size_t q = 0; q < pml.size(); ++q)
     for (int c = 0; c < 2; ++c) copy(pml[q].psi2[c], pml[q].psi[2 + c], step3_psi_bytes(q, c), hipMemcpyDeviceToDevice);
-  copy(step3_ids, step3_ids_h.data(), step3_ids_h.size(), hipMemcpyHostToDevice);
+  copy(step3_ids, step3_ids_h.get(), static_cast<size_t>(total), hipMemcpyHostToDevice);
   const std::vector<float> tab32(step3_tab_h.begin(), step3_tab_h.end());
   copy(step3_tab, plan.precision == XF_FP64 ? static_cast<const void*>(step3_tab_h.data()) : tab32.data(), step3_lds(),
        hipMemcpyHostToDevice);
