@@ -361,7 +361,10 @@ enum xf_tile_flags {
   XF_TILE_SET = 256      /* the other bits are explicit, not auto        */
 };
 
-/* Per-kernel device time accumulated by xf_run while plan.timing != 0. */
+/* Per-kernel device time accumulated by xf_run while plan.timing != 0.  The
+ * one-pass 3-D step is one launch for H and E: its time is in yee_e_ms, with
+ * the TF/SF corrections it makes; the H pass's and tfsf_ms' intervals around
+ * it are empty, and yee_h_launches counts the steps all the same. */
 typedef struct xf_timing {
   double step_ms;        /* wall-clock (events) of the whole run / steps */
   double yee_h_ms;       /* sum over launches of the H-pass kernel        */
@@ -462,10 +465,12 @@ int xf_autotune(xf_handle* h, int32_t trial_steps, xf_tuning* best);
 
 /* ---- Batches: many independent 3-D scenes of uneven sizes stepped
  * together (no reference counterpart; the reference runs one
- * SimulationHD per scene).  Every step is one persistent launch of the H
- * kernel over the tiles of all grids, one batched TFSF launch, one
- * persistent E launch, one batched TFSF + NF2FF launch; with
- * plan.use_graph a step is captured once as a hipGraph and replayed.
+ * SimulationHD per scene).  Every step is one launch of the one-pass step
+ * over the blocks of all grids where every one has its form, else one
+ * persistent launch of the H kernel over the tiles of all grids, one batched
+ * TFSF launch, one persistent E launch and one batched TFSF launch; then one
+ * batched NF2FF launch.  With plan.use_graph a step is captured once as a
+ * hipGraph (once from each set of fields in one pass) and replayed.
  * All scenes share plan.precision, the current step and the time axis;
  * ADE media and 2-D grids are not accepted (XF_ERR_UNSUPPORTED). */
 typedef struct xf_batch xf_batch;

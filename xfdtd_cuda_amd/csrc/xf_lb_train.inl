@@ -135,8 +135,9 @@ struct LbRaw {
 // a lane a column.  A butterfly over the wave for each of the 1505 parameters,
 // as before, is some 18000 dependent cross-lane operations a 64 samples:
 // 400 000 samples took 2712 us, now 230 (with k_lb_reduce 2830 and 239).
-// Bound: the forward and backward passes' VALU work, ~5000 instructions a
-// wave and 64 samples.
+// Bound: latency.  318 registers leave a wave a SIMD, so that nothing hides
+// the LDS reads of the weights and the staged rows (some 770 a wave and 64
+// samples) between the ~5000 VALU instructions, about half of the time.
 typedef double lb_d4 __attribute__((ext_vector_type(4)));
 constexpr int kLbPad = XF_LB_HID + 1;  // floats of a staged row: no two rows of a 4-sample step in the same banks
 

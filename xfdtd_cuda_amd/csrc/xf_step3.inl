@@ -26,8 +26,11 @@
 // 3.9 ms; with CPML, TF/SF and the surface sums 3.77 ms a step (two passes:
 // 4.73 ms).  A block that CPML or a TF/SF face crosses is bound by its waves'
 // chains of dependent scalar, LDS and psi accesses instead, two blocks a CU
-// to hide them (123 to 128 VGPRs in FP64): 148^3 FP64 takes 167 us a step
-// (two passes: 204), 253^3 FP32 414 (419).  Tiles of 6 to 14 rows and 9 to
+// to hide them (127 VGPRs in FP64, 96 in FP32), and by the scalars themselves:
+// all 106 SGPRs are in use and some 60 more values live in vector lanes, read
+// back lane by lane, beside a face's descriptor loaded at every plane.  156^3
+// FP64 takes 161 us a step (two passes: 191), 253^3 FP32 423 (417), FP16 430
+// (480); where the two passes are faster they run (Engine::step3_pays).  Tiles of 6 to 14 rows and 9 to
 // 54 planes a chunk measured within 3 % of each other; loads two planes ahead
 // gained FP64 nothing and cost FP32 its third block a CU (443 -> 497 us on
 // 320^3 without CPML); other block orders (contiguous ranges per XCD, the
@@ -99,7 +102,9 @@ __device__ __forceinline__ typename Store<S>::C step3_lds(const unsigned char* r
 // 16 bytes a lane from global memory to LDS at lds + 16 * lane, with no
 // register in between.  Counts on vmcnt like a load, in order; the compiler
 // does not see it, so the one wave that issues it waits for it itself (the
-// loads it issues after it and uses a plane before are enough).
+// loads it issues after it and uses a plane before are enough).  m0 cannot be
+// named as clobbered: the compiler reserves it and writes it right before each
+// use of its own.
 __device__ __forceinline__ void step3_dma16(const unsigned char* g, unsigned lds) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory");
 }

@@ -561,9 +561,10 @@ def _tuning_dict(t: XfTuning) -> dict:
 
 class Batch:
     """Many independent 3-D scenes stepped together by the engine's batched
-    kernels (xf_batch_* of include/xfdtd_hip.h): one persistent launch per
-    Yee pass over the tiles of every grid, one launch for all TFSF faces and
-    one for all NF2FF boxes per step, optionally replayed as a hipGraph."""
+    kernels (xf_batch_* of include/xfdtd_hip.h): one launch of the one-pass
+    step over the blocks of every grid, or one persistent launch per Yee pass
+    over their tiles and one for all TFSF faces, and one launch for all NF2FF
+    boxes per step, optionally replayed as a hipGraph."""
 
     def __init__(self, sims, precision: str = "fp64", use_graph: bool = False,
                  timing: bool = False, device: int = 0, watchdog: int = 0):
