@@ -523,7 +523,7 @@ def _rcs_cut(sim, phi: float, n: int = 360) -> np.ndarray:
 
 
 def batch_far_field(args, prec: str, w16) -> dict:
-    """The north star's accuracy condition for the batch: every grid of the
+    """The accuracy condition of the batch: every grid of the
     batch run to the end (`--full-steps`) in `prec` and in FP64 (bit-identical
     to the oracle), and the same spheres bounded by the learned 2-cell layer
     instead of the 8-cell CPML; RCS (xz and yz cuts at 1 GHz) relative L2
