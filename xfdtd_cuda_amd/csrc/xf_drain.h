@@ -14,10 +14,10 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstdlib>
+#include <exception>
 #include <functional>
 #include <memory>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <utility>
 #include <vector>
@@ -29,6 +29,7 @@ namespace xf {
 class StagePool {
  public:
   static constexpr size_t kSlot = size_t(16) << 20;
+  StagePool() { free_.reserve(kKept); }  // give() allocates nothing
   static std::shared_ptr<StagePool> shared() {
     static std::mutex m;
     static std::weak_ptr<StagePool> pool;
@@ -77,9 +78,10 @@ class Crew {
  public:
   explicit Crew(int n) {
     try {
+      threads_.reserve(static_cast<size_t>(n));
       for (int q = 1; q < n; ++q) threads_.emplace_back([this] { loop(); });
-    } catch (const std::system_error&) {
-      // fewer threads
+    } catch (const std::exception&) {
+      // no thread or no memory for one: fewer threads
     }
   }
   ~Crew() {
@@ -142,15 +144,16 @@ class Drain {
   // most: the largest piece that cannot be cut; all: bytes in total.
   Drain(std::shared_ptr<StagePool> pool, hipStream_t stream, size_t most, size_t all)
       : pool_(std::move(pool)), stream_(stream) {
+    // what may throw comes before the slots, which only the destructor gives back
+    const int cpus = std::max(1, static_cast<int>(std::thread::hardware_concurrency()));
+    // a thread's start is worth it from about 2 MiB of conversion on
+    crew_ = std::make_unique<Crew>(static_cast<int>(
+        std::min<size_t>(std::min(cpus, 16), std::max<size_t>(1, all / (size_t(2) << 20)))));
     // Pinning two slots takes some milliseconds, which a download pays back
     // from about kPinFrom bytes on; a smaller one goes through ordinary memory.
     if (all >= kPinFrom && most <= StagePool::kSlot) pinned_ = pool_->take();
     slot_ = pinned_ ? StagePool::kSlot : std::max(most, std::min(all, StagePool::kSlot));
     base_ = static_cast<unsigned char*>(pinned_ ? pinned_ : std::malloc(2 * slot_));
-    const int cpus = std::max(1, static_cast<int>(std::thread::hardware_concurrency()));
-    // a thread's start is worth it from about 2 MiB of conversion on
-    crew_ = std::make_unique<Crew>(static_cast<int>(
-        std::min<size_t>(std::min(cpus, 16), std::max<size_t>(1, all / (size_t(2) << 20)))));
   }
   ~Drain() {
     for (hipEvent_t& e : event_)

@@ -1124,8 +1124,8 @@ void host_parallel_for(int64_t n, F fn) {
       const int64_t t = started;
       pool.emplace_back([&, t] { fn(n * t / nth, n * (t + 1) / nth); });
     }
-  } catch (const std::system_error&) {
-    // a thread could not start: its range and the rest run on this thread
+  } catch (const std::exception&) {
+    // no thread or no memory for one: its range and the rest run on this thread
   }
   for (int64_t t = started; t < nth; ++t) fn(n * t / nth, n * (t + 1) / nth);
   for (auto& th : pool) th.join();
@@ -1198,7 +1198,7 @@ int Engine::unpack_fields(Drain& out) {
       const int64_t planes = std::min(step, a.shape[0] - p0);
       double* to = a.data + p0 * nj * nk;
       // rows [lo, hi) of these planes
-      auto put = [=, this](const unsigned char* from, int64_t lo, int64_t hi) {
+      auto put = [=](const unsigned char* from, int64_t lo, int64_t hi) {
         for (int64_t r = lo; r < hi; ++r) {
           const int64_t at = dim == 3 ? r / nj * sx + r % nj * sy : r / nj * sx + r % nj;
           double* const o = to + r * nk;
