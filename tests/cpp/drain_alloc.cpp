@@ -64,7 +64,7 @@ static int download(const std::shared_ptr<xf::StagePool>& pool, const std::vecto
   fail_at = k;
   int ok = 1;
   try {
-    xf::Drain out(pool, nullptr, 1 << 16, all);
+    xf::Drain out(pool, nullptr, 1 << 16, all, size_t(8) << 20);
     if (out.open() != hipSuccess) std::abort();
     const size_t part = from.size() / 8;
     for (size_t q = 0; q < 8; ++q) {
@@ -91,7 +91,7 @@ static int download(const std::shared_ptr<xf::StagePool>& pool, const std::vecto
 int main() {
   std::vector<double> from(8 * 4096), to(from.size());
   for (size_t q = 0; q < from.size(); ++q) from[q] = static_cast<double>(q) + 0.5;
-  for (const size_t all : {size_t(8) << 20, size_t(64) << 20}) {  // ordinary and pinned slots, threads in both
+  for (const size_t all : {size_t(2) << 20, size_t(64) << 20}) {  // ordinary and pinned slots, threads in both
     auto pool = std::make_shared<xf::StagePool>();
     if (download(pool, from, to, all, -1) != 1) return 2;
     const long live0 = live, pinned0 = pinned;

@@ -807,14 +807,15 @@ int Batch::download() {
   XF_HIP(hipStreamSynchronize(stream));
   if (inst.empty()) return XF_OK;
   // one pass through the staging slots for every grid
-  size_t most = 0, all = 0;
+  size_t most = 0, all = 0, work = 0;
   for (auto& h : inst) {
     XF_HIP(hipStreamSynchronize(h->eng.stream));
     most = std::max(most, h->eng.plane_bytes());
     all += h->eng.drain_bytes();
+    work += h->eng.drain_work();
   }
   {
-    Drain out(inst[0]->eng.stages, stream, most, all);
+    Drain out(inst[0]->eng.stages, stream, most, all, work);
     XF_HIP(out.open());
     for (auto& h : inst) XF_TRY(h->eng.drain(out));
     XF_HIP(out.finish());

@@ -141,18 +141,23 @@ class Drain {
  public:
   using Put = std::function<void(const unsigned char*, int64_t, int64_t)>;
 
-  // most: the largest piece that cannot be cut; all: bytes in total.
-  Drain(std::shared_ptr<StagePool> pool, hipStream_t stream, size_t most, size_t all)
+  // most: the largest piece that cannot be cut; all: bytes in total; work: the
+  // conversion, in bytes of the caller's memory that a copy writes as fast.
+  Drain(std::shared_ptr<StagePool> pool, hipStream_t stream, size_t most, size_t all, size_t work)
       : pool_(std::move(pool)), stream_(stream) {
     // what may throw comes before the slots, which only the destructor gives back
     const int cpus = std::max(1, static_cast<int>(std::thread::hardware_concurrency()));
     // a thread's start is worth it from about 2 MiB of conversion on
     crew_ = std::make_unique<Crew>(static_cast<int>(
-        std::min<size_t>(std::min(cpus, 16), std::max<size_t>(1, all / (size_t(2) << 20)))));
-    // Pinning two slots takes some milliseconds, which a download pays back
-    // from about kPinFrom bytes on; a smaller one goes through ordinary memory.
+        std::min<size_t>(std::min(cpus, 16), std::max<size_t>(1, work / (size_t(2) << 20)))));
+    // Pinning two slots takes 0.3 to 1.5 ms, the first time in a process, which a
+    // download pays back from about kPinFrom bytes on; a smaller one goes through
+    // ordinary memory, where 20 to 40 MB took 7 to 10 ms (in pinned slots 1.1 to
+    // 2).  A download of up to 64 MiB fills four slots, so that copies and
+    // conversion overlap.
     if (all >= kPinFrom && most <= StagePool::kSlot) pinned_ = pool_->take();
-    slot_ = pinned_ ? StagePool::kSlot : std::max(most, std::min(all, StagePool::kSlot));
+    slot_ = pinned_ ? std::max(most, std::min(std::max(all / 4, size_t(1) << 20), StagePool::kSlot))
+                    : std::max(most, std::min(all, StagePool::kSlot));
     base_ = static_cast<unsigned char*>(pinned_ ? pinned_ : std::malloc(2 * slot_));
   }
   ~Drain() {
@@ -236,7 +241,7 @@ class Drain {
     return hipSuccess;
   }
 
-  static constexpr size_t kPinFrom = size_t(48) << 20, kUnit = size_t(256) << 10;
+  static constexpr size_t kPinFrom = size_t(4) << 20, kUnit = size_t(256) << 10;
   std::shared_ptr<StagePool> pool_;
   hipStream_t stream_;
   void* pinned_ = nullptr;
