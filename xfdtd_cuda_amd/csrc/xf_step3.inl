@@ -24,7 +24,10 @@
 // without CPML takes 3.0 ms for 15.1 GB, 5.0 TB/s, where a plain copy of six
 // such arrays into six others reaches 5.4 TB/s and the two-pass kernels take
 // 3.9 ms; with CPML, TF/SF and the surface sums 3.77 ms a step (two passes:
-// 4.73 ms).  A block that CPML or a TF/SF face crosses is bound by its waves'
+// 4.73 ms).  By the counters the latter is 14.5 GB read past the L2s for 8.9
+// that a step needs, since blocks that share halo rows and columns run on
+// different XCDs, and 8.1 GB written: 22.7 GB at 94 % of the rate of a copy of
+// one array.  A block that CPML or a TF/SF face crosses is bound by its waves'
 // chains of dependent scalar, LDS and psi accesses instead, two blocks a CU
 // to hide them (127 VGPRs in FP64, 96 in FP32), and by the scalars themselves:
 // all 106 SGPRs are in use and some 60 more values live in vector lanes, read
