@@ -33,8 +33,9 @@
 // all 106 SGPRs are in use and some 60 more values live in vector lanes, read
 // back lane by lane, beside a face's descriptor loaded at every plane.  156^3
 // FP64 takes 161 us a step (two passes: 191), 253^3 FP32 423 (417), FP16 430
-// (480); where the two passes are faster they run (Engine::step3_pays).  Tiles of 6 to 14 rows and 9 to
-// 54 planes a chunk measured within 3 % of each other; loads two planes ahead
+// (480); where the two passes are faster they run (Engine::step3_pays).  Tiles
+// of 6 to 14 rows and 9 to 54 planes a chunk measured within 3 % of each other;
+// loads two planes ahead
 // gained FP64 nothing and cost FP32 its third block a CU (443 -> 497 us on
 // 320^3 without CPML); other block orders (contiguous ranges per XCD, the
 // grid's end tiles first) lose 3 to 15 %, because neighbours in j, which read
